@@ -62,6 +62,12 @@ int gemv_t16_launch(const void* tiles, const void* tile_scales, const float* x, 
 // advance[0] += delta afterwards in the same kernel.
 int argmax_final_launch(const ArgBest* partials, int n, int32_t* out, int32_t* advance, int delta, hipStream_t st);
 
+// q4_linear for a few rows of x in one launch (q4_rows.hip), for the sizes q4_rows_takes; arguments
+// checked by the caller (K % 64 == 0, group % 32 == 0, M <= 32).
+bool q4_rows_takes(int64_t M, int64_t K);
+int q4_rows_launch(const float* x, int64_t M, const int32_t* qw, const uint16_t* sc, float* y, const float* res,
+                   int64_t N, int64_t K, int group, hipStream_t st);
+
 // K split of a prefill projection: n_split workgroups per output tile, nk_split 64-k stages each.
 struct LinearSplit {
   int n_split, nk_split;

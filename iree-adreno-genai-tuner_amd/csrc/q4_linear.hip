@@ -932,6 +932,7 @@ constexpr int kNumLinWs = sizeof(kLinWsTiles) / sizeof(kLinWsTiles[0]);
 
 int q4_linear_launch(const float* x, int64_t M, const int32_t* qw, const uint16_t* sc, float* y, const float* res,
                      int64_t N, int64_t K, int group, int cfg, hipStream_t st) {
+  if (cfg < 0 && q4_rows_takes(M, K)) return q4_rows_launch(x, M, qw, sc, y, res, N, K, group, st);
   int ti = cfg;
   if (ti < 0 || ti > 2) {
     ti = 2;
@@ -1100,8 +1101,10 @@ int q4_linear_planes_swiglu(const uint16_t* xh, const uint16_t* xl, int64_t M, c
 // the K-split partials.
 int q4_linear_ws_launch(const float* x, int64_t M, const int32_t* qw, const uint16_t* sc, float* y, const float* res,
                         int64_t N, int64_t K, int group, void* ws, size_t ws_bytes, hipStream_t st) {
-  // the pipelined kernel indexes groups by shifts: other group sizes take the workspace-free kernel
-  if (group & (group - 1)) return q4_linear_launch(x, M, qw, sc, y, res, N, K, group, -1, st);
+  // the pipelined kernel indexes groups by shifts: other group sizes take the workspace-free kernel,
+  // as do few rows (Q4_DBG_LINEAR_TILE set: the pipelined kernel)
+  if ((group & (group - 1)) || (q4_rows_takes(M, K) && !debug_set(Q4_DBG_LINEAR_TILE)))
+    return q4_linear_launch(x, M, qw, sc, y, res, N, K, group, -1, st);
   uint16_t* xh = static_cast<uint16_t*>(ws);
   uint16_t* xl = xh + M * K;
   const int64_t chunks = M * K / 8;

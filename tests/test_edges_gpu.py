@@ -40,3 +40,32 @@ def test_quantize_non_finite_same_on_both_paths(dev, group):
     w[0, 3], w[1, 70], w[2, 500], w[3, :] = float("inf"), float("nan"), float("-inf"), float("nan")
     a, b = ops.quantize_q4(w, group), ops.quantize_q4(misaligned(w), group)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1].view(torch.int16), b[1].view(torch.int16))
+
+
+def linear_case(dev, M, N, K, group, seed):
+    g = torch.Generator().manual_seed(seed)
+    qw, sc = R.quantize_q4(torch.randn(N, K, generator=g) * 0.02, group)
+    x, res = torch.randn(M, K, generator=g), torch.randn(M, N, generator=g)
+    w = R.dequantize_q4(qw, sc, group).double()
+    ref = x.double() @ w.t() + res.double()
+    # x = hi + lo up to 2^-22 |x|; fp32 sums of at most two adds per 32 k, a scale per group and the
+    # waves' and residual's adds, each rounding by 2^-24 of a partial sum that sum |x w| + |res| bounds
+    bound = ((x.double().abs() @ w.abs().t()) + res.double().abs()) * (2.0 ** -22 + (K / 16 + K / group + 32) * 2.0 ** -24)
+    return x.to(dev), qw.to(dev), sc.to(dev), res.to(dev), ref, bound
+
+
+@pytest.mark.parametrize("M,N,K,group", [(2, 1, 64, 32), (16, 15, 192, 64), (17, 33, 96 * 4, 96), (9, 4097, 256, 128),
+                                         (32, 4112, 128, 32), (3, 8193, 192, 32), (31, 8208, 384, 384), (1, 16, 4160, 64),
+                                         (32, 48, 4096, 128), (16, 17, 8192, 256), (33, 48, 4096, 128), (17, 16, 4160, 32)])
+def test_linear_few_rows(dev, M, N, K, group):
+    """The one-launch kernel for few rows at the edges of its column counts (16, 32 and 64 per workgroup),
+    K remainders (64 of a 128-k step, fewer steps than waves), groups (any multiple of 32) and its
+    largest M, and the sizes just past its rule; the residual aliasing y, with and without a workspace."""
+    x, qw, sc, res, ref, bound = linear_case(dev, M, N, K, group, M * 1000 + N)
+    for fn in (ops.q4_linear, ops.q4_linear_ws):
+        y = torch.full((M, N), float("nan"), device=dev)
+        fn(x, qw, sc, group, out=y)
+        assert ((y.cpu().double() - (ref - res.cpu().double())).abs() <= bound).all(), (fn, M, N, K, group)
+        h = res.clone()
+        fn(x, qw, sc, group, residual=h, out=h)
+        assert ((h.cpu().double() - ref).abs() <= bound).all(), (fn, M, N, K, group)
