@@ -200,8 +200,8 @@ int q4_linear(const float* x, int64_t M, const int32_t* qweight, const uint16_t*
 /* Workspace bytes q4_linear_ws needs for M rows of K: the fp16 hi and lo planes of x (4 * M * K). */
 int q4_linear_workspace_bytes(int64_t M, int64_t K, size_t* bytes);
 
-/* Workspace bytes with which q4_linear_ws also splits the reduction over K for this shape (a chunk of
- * M <= 256 rows whose output tiles alone would leave compute units idle): the planes, rounded up to
+/* Workspace bytes with which q4_linear_ws also splits the reduction over K for this shape (where its
+ * output tiles alone would leave compute units idle): the planes, rounded up to
  * 256 bytes, plus n_split * M * N fp32 partials; equal to q4_linear_workspace_bytes(M, K) where no
  * split applies. */
 int q4_linear_ws_split_bytes(int64_t M, int64_t N, int64_t K, int group, size_t* bytes);

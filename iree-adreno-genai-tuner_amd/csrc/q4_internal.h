@@ -75,6 +75,8 @@ struct LinearSplit {
 LinearSplit linear_split_plan(int64_t M, int64_t N, int64_t K, int group);
 // bytes of K-split partials q4_linear_planes uses for this shape (0: it takes no K split)
 size_t linear_split_part_bytes(int64_t M, int64_t N, int64_t K, int group);
+// the same for q4_linear_ws, which may split K past 256 rows too
+size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group);
 
 // q4_linear_ws's GEMM on given planes (power-of-two group); with `part` (at least
 // linear_split_part_bytes, 16-byte aligned) it may split K and reduce the partials in a second kernel.

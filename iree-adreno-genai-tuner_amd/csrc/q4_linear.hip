@@ -17,6 +17,8 @@
 #include "q4_common.h"
 #include "q4_internal.h"
 
+#include <algorithm>
+#include <cstdint>
 #include <cstdlib>
 
 namespace q4 {
@@ -883,12 +885,12 @@ struct LinWsTile {
 // 128x128, 128x256, 64x512), 64x64 waves on 128x256, k-split 2-wave and 64x64 / 128x64 / 32x96 /
 // 32x128 / 32x160 variants.
 constexpr LinWsTile kLinWsTiles[] = {
-    {64, 64, 2, 2, 4, 1},    // 0: 4 waves of 32x32, 4 stages (77 KB)
-    {32, 64, 1, 2, 4, 2},    // 1: 4 waves: 2 tiles of 32x32, each k-split over 2 waves (52 KB)
-    {64, 256, 2, 4, 4, 1, true},  // 2: 8 waves of 32x64, software-pipelined: one workgroup per CU for
-                                  // 256-row chunks, and the K split
+    {32, 64, 1, 2, 4, 2},          // 0: 4 waves: 2 tiles of 32x32, each k-split over 2 waves (52 KB)
+    {64, 256, 2, 4, 4, 1, true},   // 1: 8 waves of 32x64, software-pipelined: one workgroup per CU for
+                                   // 256-row chunks, and the K split
+    {128, 256, 2, 4, 3, 1, true},  // 2: 8 waves of 64x64, 3 stages (127 KB), software-pipelined: many rows
 };
-constexpr int kSplitTile = 2;  // the K-split tile (linear_split_plan) and the SwiGLU-epilogue tile
+constexpr int kSmallTile = 0, kSplitTile = 1, kLargeTile = 2;  // kSplitTile: also the SwiGLU-epilogue tile
 using LinWsFn = void (*)(const uint16_t*, const uint16_t*, const int32_t*, const uint16_t*, float*, const float*, int,
                          int, int, int, int, int, int, float*, int, int);
 template <int I>
@@ -896,10 +898,10 @@ constexpr LinWsFn lin_ws_fn() {
   constexpr LinWsTile t = kLinWsTiles[I];
   return q4_linear_ws_kernel<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks, 0, t.pipe>;
 }
-// the K-split / SwiGLU tile with the weight in the T16 layout (EPI 0 or 1)
-template <int EPI>
+// a pipelined tile with the weight in the T16 layout (EPI 0 or 1)
+template <int EPI, int I>
 constexpr LinWsFn lin_ws_t16_fn() {
-  constexpr LinWsTile t = kLinWsTiles[kSplitTile];
+  constexpr LinWsTile t = kLinWsTiles[I];
   return q4_linear_ws_kernel<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks, EPI, true, true>;
 }
 template <int I>
@@ -908,10 +910,13 @@ constexpr size_t lin_ws_lds() {
   return LinWsCfg<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks>::kLds;
 }
 constexpr LinWsFn kLinWsFns[] = {lin_ws_fn<0>(), lin_ws_fn<1>(), lin_ws_fn<2>()};
+constexpr LinWsFn kLinWsT16Fns[] = {nullptr, lin_ws_t16_fn<0, kSplitTile>(), lin_ws_t16_fn<0, kLargeTile>()};
 constexpr size_t kLinWsLds[] = {lin_ws_lds<0>(), lin_ws_lds<1>(), lin_ws_lds<2>()};
-static_assert(kLinWsTiles[kSplitTile].pipe && kLinWsTiles[kSplitTile].ks == 1, "the T16 variants need the pipelined loop");
+static_assert(kLinWsTiles[kSplitTile].pipe && kLinWsTiles[kSplitTile].ks == 1 && kLinWsTiles[kLargeTile].pipe &&
+                  kLinWsTiles[kLargeTile].ks == 1,
+              "the T16 variants need the pipelined loop");
 
-// A T16 source the K-split tile can read: both pointers, a group the layout takes, whole 16-row tiles
+// A T16 source the pipelined tiles can read: both pointers, a group the layout takes, whole 16-row tiles
 // for the paired orders, 16-byte aligned tiles (Q4_DBG_PREFILL_REF_LAYOUT set: the reference layout).
 bool t16_usable(const T16Src* t, int64_t N, int group, int pairing_needed) {
   if (!t || !t->tiles || !t->scales || debug_flag(Q4_DBG_PREFILL_REF_LAYOUT)) return false;
@@ -1001,71 +1006,117 @@ size_t linear_split_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
   return p.n_split > 1 ? static_cast<size_t>(p.n_split) * M * N * sizeof(float) : 0;
 }
 
+namespace {
+// A tile entry with its K split.
+struct LinPlan {
+  int tile;
+  LinearSplit split;
+  size_t part_bytes(int64_t M, int64_t N) const {
+    return split.n_split > 1 ? static_cast<size_t>(split.n_split) * M * N * sizeof(float) : 0;
+  }
+};
+
+// Estimated time (us) of `wgs` workgroups of `steps` 64-k stages each on tile entry `ti`: rounds of at most
+// kRound workgroups, whose stage time grows with how many of them run (the matrix cores' clock and the
+// L2 are shared). Constants fitted to one MI355X, graph replays over rotated weights, group 128 | 32:
+//   64x256 (8 waves of 32x64):   48 workgroups 0.86 | 1.29 us a stage, 160 1.03 | 1.41, 256 1.16 | 1.60
+//   128x256 (8 waves of 64x64):  40 workgroups 1.37 | 2.13, 128 1.58 | 2.29, 256 1.92 | 2.63
+//   32x64 (three per CU):        480 workgroups 0.56 | 0.63, 768 0.83 | 0.92
+double tile_time(int ti, int64_t wgs, int64_t steps, int group) {
+  struct Rate {
+    double fixed, a, b;
+    int round;
+  };
+  constexpr Rate kRates[2][3] = {{{6.0, 0.30, 0.00070, 768}, {7.0, 0.82, 0.00133, 256}, {8.0, 1.28, 0.0025, 256}},
+                                 {{6.0, 0.36, 0.00073, 768}, {7.0, 1.23, 0.00145, 256}, {8.0, 2.03, 0.0023, 256}}};
+  const Rate& r = kRates[group >= 128 ? 0 : 1][ti];
+  double t = r.fixed;
+  for (; wgs > 0; wgs -= r.round) t += steps * (r.a + r.b * static_cast<double>(std::min<int64_t>(wgs, r.round)));
+  return t;
+}
+
+// The cheapest tile by tile_time, with a K split (pipelined tiles; whole groups, at least four stages, at
+// most eight splits) where the planes may be followed by up to `part_bytes` of partials: their write and
+// read cost 8 S M N bytes at 4.5 TB/s and the reduce launch 2.5 us. Against the 64x64 and 32x64 tiles that
+// ran all of these before (us, with the x split): 512x5120x3072 78.8 -> 52.4, 512x16384x3072 197 -> 100
+// (group 32: 241 -> 135), 1024x5120x3072 127 -> 83, 1024x16384x3072 375 -> 190.
+LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes) {
+  const int64_t nk = K / 64, gst = group > 64 ? group / 64 : 1;
+  LinPlan best{kSmallTile, {1, 0}};
+  double best_t = 0.0;
+  for (int ti = 0; ti < kNumLinWs; ++ti) {
+    const LinWsTile& t = kLinWsTiles[ti];
+    const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    for (int64_t want = 1; want <= (t.pipe ? 8 : 1); ++want) {
+      int64_t nk_s = (nk + want - 1) / want;
+      nk_s = (nk_s + gst - 1) / gst * gst;
+      const int64_t S = (nk + nk_s - 1) / nk_s;
+      if (S != want || (S > 1 && (nk_s < 4 || static_cast<size_t>(S) * M * N * sizeof(float) > part_bytes))) continue;
+      double us = tile_time(ti, tiles * S, nk_s, group);
+      if (S > 1) us += 2.5 + 8e-6 / 4.5 * static_cast<double>(S * M * N);
+      if ((ti == 0 && S == 1) || us < best_t) {
+        best_t = us;
+        best = LinPlan{ti, {static_cast<int>(S), S > 1 ? static_cast<int>(nk_s) : 0}};
+      }
+    }
+  }
+  return best;
+}
+
+// The rule: chunks of at most 256 rows with room for their partials take linear_split_plan where it
+// splits; everything else the cheapest tile.
+LinPlan linear_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes) {
+  const LinearSplit sp = linear_split_plan(M, N, K, group);
+  if (sp.n_split > 1 && part_bytes >= linear_split_part_bytes(M, N, K, group)) return LinPlan{kSplitTile, sp};
+  return tile_plan(M, N, K, group, M > 256 ? part_bytes : 0);
+}
+}  // namespace
+
+// Bytes of partials with which q4_linear_planes takes its fastest plan, outside the model step too
+// (there linear_split_part_bytes: no split past 256 rows).
+size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
+  if (M <= 256) return linear_split_part_bytes(M, N, K, group);
+  return tile_plan(M, N, K, group, SIZE_MAX).part_bytes(M, N);
+}
+
 // The pipelined GEMM on x given as fp16 (hi, lo) planes (store_x_planes layout, [M, K] each);
-// power-of-two groups only. Tile rule from a sweep of every entry over the 3B prefill shapes at
-// M = 128, 256 and 1024 (graph replays on one MI355X): with a partial buffer `part` of at least
-// linear_split_part_bytes, the K-split 64x256 tile where linear_split_plan gives a split (every M <= 256
-// chunk of the 3072-, 5120- and 8192-wide projections), then linear_reduce_kernel; otherwise the 32x64
-// k-split tile while it gives at most 768 workgroups, else 64x64. Q4_DBG_LINEAR_TILE overrides (no K split).
+// power-of-two groups only. linear_plan picks the tile and, with a partial buffer `part` that holds it,
+// the K split, whose partials linear_reduce_kernel adds. Q4_DBG_LINEAR_TILE overrides (no K split).
 int q4_linear_planes(const uint16_t* xh, const uint16_t* xl, int64_t M, const int32_t* qw, const uint16_t* sc,
                      float* y, const float* res, int64_t N, int64_t K, int group, hipStream_t st, float* part,
                      size_t part_bytes, int* deferred, const T16Src* t16) {
   if (int e = planes_args(xh, xl, M, qw, sc, N, K, group)) return e;
   if (!y) return Q4_ERR_NULL;
   if (deferred) *deferred = 0;
-  int ti = -1;
+  // what the partials and linear_reduce_kernel need: whole float4s, 16-byte alignment, 32-bit indexes
+  const bool can_split = part && (M * N) % 4 == 0 && aligned(part, 16) && aligned(y, 16) && (!res || aligned(res, 16));
+  LinPlan plan = linear_plan(M, N, K, group, can_split ? std::min<size_t>(part_bytes, size_t{1} << 33) : 0);
   const int ov = debug_override(Q4_DBG_LINEAR_TILE);
-  if (ov >= 0 && ov < kNumLinWs) ti = ov;
-  const LinearSplit sp = linear_split_plan(M, N, K, group);
-  if (ti < 0 && part && sp.n_split > 1 && part_bytes >= linear_split_part_bytes(M, N, K, group) &&
-      (M * N) % 4 == 0 && aligned(part, 16) && aligned(y, 16) && (!res || aligned(res, 16)) &&
-      static_cast<int64_t>(sp.n_split) * M * N < (int64_t{1} << 31)) {
-    constexpr int T = kSplitTile;
-    const LinWsTile& t = kLinWsTiles[T];
-    const int tiles_n = static_cast<int>((N + t.bn - 1) / t.bn);
-    const int tiles = static_cast<int>((M + t.bm - 1) / t.bm) * tiles_n;
-    const bool use_t16 = t16_usable(t16, N, group, -1);
-    const LinWsFn fn = use_t16 ? lin_ws_t16_fn<0>() : kLinWsFns[T];
-    if (kLinWsLds[T] > 64 * 1024) {
-      Q4_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       static_cast<int>(kLinWsLds[T])));
-    }
-    hipLaunchKernelGGL(fn, dim3(tiles * sp.n_split), dim3(64 * t.wm * t.wn * t.ks), kLinWsLds[T], st, xh, xl,
-                       use_t16 ? static_cast<const int32_t*>(t16->tiles) : qw, use_t16 ? t16->scales : sc, y, res,
-                       (int)M, (int)N, (int)K, group, tiles_n, sp.n_split, sp.nk_split, part,
-                       use_t16 ? t16->pairing : 0, use_t16 ? t16->head_dim : 0);
-    if (int e = launch_status()) return e;
-    if (deferred) {
-      *deferred = sp.n_split;
-      return Q4_OK;
-    }
-    const int64_t n4 = M * N / 4;
-    hipLaunchKernelGGL(linear_reduce_kernel, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, st,
-                       reinterpret_cast<const float4*>(part), reinterpret_cast<const float4*>(res),
-                       reinterpret_cast<float4*>(y), n4, sp.n_split);
-    return launch_status();
-  }
-  // Rule from a sweep at M = 128, 256, 1024: the 32x64 k-split tile while it gives <= 768 workgroups,
-  // else 64x64; and 64x256 when, at M <= 256, it alone gives one workgroup per CU (the gate/up
-  // projection of a 256-row chunk: 256x16384x3072 82 -> 69 us, x re-read over 4x fewer column tiles).
-  if (ti < 0) {
-    const int64_t wide = ((M + 63) / 64) * ((N + 255) / 256);
-    if (M <= 256 && wide >= 256) ti = kSplitTile;
-    else ti = ((M + 31) / 32) * ((N + 63) / 64) <= 768 ? 1 : 0;
-  }
+  if (ov >= 0 && ov < kNumLinWs) plan = LinPlan{ov, {1, 0}};
+  const int ti = plan.tile, S = plan.split.n_split;
   const LinWsTile& t = kLinWsTiles[ti];
   const int tiles_n = static_cast<int>((N + t.bn - 1) / t.bn);
   const int tiles = static_cast<int>((M + t.bm - 1) / t.bm) * tiles_n;
-  const bool use_t16 = ti == kSplitTile && t16_usable(t16, N, group, -1);
-  const LinWsFn fn = use_t16 ? lin_ws_t16_fn<0>() : kLinWsFns[ti];
+  const bool use_t16 = t.pipe && t16_usable(t16, N, group, -1);
+  const LinWsFn fn = use_t16 ? kLinWsT16Fns[ti] : kLinWsFns[ti];
   if (kLinWsLds[ti] > 64 * 1024) {
     Q4_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                      static_cast<int>(kLinWsLds[ti])));
   }
-  hipLaunchKernelGGL(fn, dim3(tiles), dim3(64 * t.wm * t.wn * t.ks), kLinWsLds[ti], st, xh, xl,
+  hipLaunchKernelGGL(fn, dim3(tiles * S), dim3(64 * t.wm * t.wn * t.ks), kLinWsLds[ti], st, xh, xl,
                      use_t16 ? static_cast<const int32_t*>(t16->tiles) : qw, use_t16 ? t16->scales : sc, y, res, (int)M,
-                     (int)N, (int)K, group, tiles_n, 1, 0, nullptr, use_t16 ? t16->pairing : 0,
-                     use_t16 ? t16->head_dim : 0);
+                     (int)N, (int)K, group, tiles_n, S, plan.split.nk_split, S > 1 ? part : nullptr,
+                     use_t16 ? t16->pairing : 0, use_t16 ? t16->head_dim : 0);
+  if (int e = launch_status()) return e;
+  if (S == 1) return Q4_OK;
+  if (deferred) {
+    *deferred = S;
+    return Q4_OK;
+  }
+  const int64_t n4 = M * N / 4;
+  hipLaunchKernelGGL(linear_reduce_kernel, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, st,
+                     reinterpret_cast<const float4*>(part), reinterpret_cast<const float4*>(res),
+                     reinterpret_cast<float4*>(y), n4, S);
   return launch_status();
 }
 
@@ -1082,7 +1133,7 @@ int q4_linear_planes_swiglu(const uint16_t* xh, const uint16_t* xl, int64_t M, c
   const int64_t wide = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
   if (!(M <= 256 && wide >= 256) || N % t.bn || (N / 2) % 32 || ol != oh + M * (N / 2)) return Q4_ERR_UNSUPPORTED;
   const bool use_t16 = t16_usable(t16, N, group, Q4_PAIR_SWIGLU);
-  const LinWsFn fn = use_t16 ? lin_ws_t16_fn<1>() : q4_linear_ws_kernel<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks, 1, t.pipe>;
+  const LinWsFn fn = use_t16 ? lin_ws_t16_fn<1, kSplitTile>() : q4_linear_ws_kernel<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks, 1, t.pipe>;
   constexpr size_t lds = LinWsCfg<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks>::kLds;
   if (lds > 64 * 1024) {
     Q4_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1149,7 +1200,7 @@ extern "C" int q4_linear_ws_split_bytes(int64_t M, int64_t N, int64_t K, int gro
   if (!bytes) return Q4_ERR_NULL;
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 || group <= 0) return Q4_ERR_SHAPE;
   const size_t planes = (static_cast<size_t>(M) * K * 4 + 255) / 256 * 256;
-  const size_t part = (group & (group - 1)) == 0 ? q4::linear_split_part_bytes(M, N, K, group) : 0;
+  const size_t part = (group & (group - 1)) == 0 ? q4::linear_plan_part_bytes(M, N, K, group) : 0;
   *bytes = part ? planes + part : static_cast<size_t>(M) * K * 4;
   return Q4_OK;
 }

@@ -157,9 +157,29 @@ def q4_linear(x, qweight, scales, group, residual=None, out=None):
     _dev(qweight, scales, x, residual, out)
     if out is None:
         out = torch.empty(m, n, dtype=torch.float32, device=x.device)
-    LIB.call("q4_linear", ptr(x), m, ptr(qweight), ptr(scales), ptr(out), ptr(residual), n, k, group,
-             stream_of(x.device))
+    ws, ws_bytes = _linear_workspace(x, m, n, k, group)
+    if ws is None:
+        LIB.call("q4_linear", ptr(x), m, ptr(qweight), ptr(scales), ptr(out), ptr(residual), n, k, group,
+                 stream_of(x.device))
+    else:
+        LIB.call("q4_linear_ws", ptr(x), m, ptr(qweight), ptr(scales), ptr(out), ptr(residual), n, k, group,
+                 ptr(ws), ws_bytes, stream_of(x.device))
     return out
+
+
+def _linear_workspace(x, m, n, k, group):
+    """(uint8 workspace, bytes) for q4_linear's tiled path, from torch's allocator on the current stream
+    (its pool keeps the block for the next call); (None, 0) where the workspace-free kernel runs: a few
+    rows, sizes the tiled path refuses, or no memory for the x planes and partials."""
+    if m <= 16 or k % 64 or group % 32 or group & (group - 1) or m * k >= 1 << 29:
+        return None, 0
+    need = q4_linear_ws_split_bytes(m, n, k, group)
+    for nbytes in (need, 4 * m * k):
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=x.device), nbytes
+        except torch.OutOfMemoryError:
+            pass
+    return None, 0
 
 
 def q4_linear_ws_split_bytes(m, n, k, group) -> int:

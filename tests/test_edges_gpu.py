@@ -69,3 +69,21 @@ def test_linear_few_rows(dev, M, N, K, group):
         h = res.clone()
         fn(x, qw, sc, group, residual=h, out=h)
         assert ((h.cpu().double() - ref).abs() <= bound).all(), (fn, M, N, K, group)
+
+
+@pytest.mark.parametrize("M,N,K,group", [(33, 40, 128, 32), (100, 515, 3072, 32), (257, 256, 256, 128), (300, 1030, 2048, 64),
+                                         (385, 260, 4096, 256), (513, 3072, 1024, 128), (640, 5120, 192, 64),
+                                         (1024, 4100, 512, 128)])
+def test_linear_many_rows(dev, M, N, K, group):
+    """q4_linear through its workspace: both pipelined tiles with ragged rows and columns, K splits past
+    256 rows, an exact-planes workspace (no split), and a residual aliasing y."""
+    x, qw, sc, res, ref, bound = linear_case(dev, M, N, K, group, M + N)
+    y = torch.full((M, N), float("nan"), device=dev)
+    ops.q4_linear(x, qw, sc, group, out=y)
+    assert ((y.cpu().double() - (ref - res.cpu().double())).abs() <= bound).all()
+    for split in (False, True):
+        h = res.clone()
+        need = ops.q4_linear_ws_split_bytes(M, N, K, group) if split else 4 * M * K
+        ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=dev)
+        ops.q4_linear_ws(x, qw, sc, group, residual=h, out=h, workspace=ws)
+        assert ((h.cpu().double() - ref).abs() <= bound).all(), split
