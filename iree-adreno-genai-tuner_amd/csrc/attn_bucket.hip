@@ -47,9 +47,13 @@ AttnPlan plan_for(int C, int n_q, int n_kv, int L) {
     const int ov = debug_override(Q4_DBG_ATTN_S);  // sweep override: keys per split (32, 64 or 128)
     if (ov == 32 || ov == 64 || ov == 128) p.S = ov;
   } else if (g <= kMfmaMaxG && !debug_flag(Q4_DBG_ATTN_GENERIC)) {
+    // Keys per split: enough for about two workgroups of four 32-row units per CU, at least 64 (128 past
+    // 256 keys): more splits only add partials to write and merge.
     p.mfma = true;
     p.CB = 32;
-    p.S = L <= 256 ? 64 : 128;
+    const int64_t wgs = static_cast<int64_t>(n_kv) * (((C + 31) / 32 * g + 3) / 4);  // per split
+    const int64_t want = std::max<int64_t>(1, 512 / wgs);
+    p.S = std::max(L <= 256 ? 64 : 128, static_cast<int>((L + 32 * want - 1) / (32 * want)) * 32);
     const int ov = debug_override(Q4_DBG_ATTN_PS);  // sweep override: keys per split (a multiple of 32, <= 512)
     if (ov != Q4_DBG_UNSET && ov >= 32 && ov <= 512 && ov % 32 == 0) p.S = ov;
   } else {
@@ -258,6 +262,11 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(
   }
 }
 
+// Weight of a split with maximum m where the largest is M; base2: the matrix-core prefill's log2 units.
+__device__ __forceinline__ float split_weight(float m, float M, bool base2) {
+  return m == -INFINITY ? 0.0f : base2 ? exp2f(m - M) : expf(m - M);
+}
+
 // Merge the splits of each (row, head), one thread per 8 dims of one (row, head): no LDS and no
 // barrier. Every (m, l) and this thread's 8 o values of the first kB splits are requested before
 // the position is read (range-checked buffer loads: zeros past the workspace), so the merge costs one
@@ -267,7 +276,8 @@ template <int HD>
 __global__ __launch_bounds__(256) void attn_combine8_kernel(const float* __restrict__ ws_ml, const float* __restrict__ ws_o,
                                                           float* __restrict__ out, int64_t rows, int n_q, int n_splits,
                                                           int S, const int32_t* __restrict__ start_p,
-                                                          uint16_t* __restrict__ xh, uint16_t* __restrict__ xl) {
+                                                          uint16_t* __restrict__ xh, uint16_t* __restrict__ xl,
+                                                          bool base2) {
   constexpr int kB = 8, D8 = HD / 8;
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -301,7 +311,7 @@ __global__ __launch_bounds__(256) void attn_combine8_kernel(const float* __restr
 #pragma unroll
   for (int e = 0; e < 8; ++e) num[e] = 0.0f;
   auto add = [&](float m, float l, const f32x4& a, const f32x4& b) {
-    const float w = m == -INFINITY ? 0.0f : expf(m - M);
+    const float w = split_weight(m, M, base2);
     den = fmaf(w, l, den);
     num[0] = fmaf(w, a.x, num[0]);
     num[1] = fmaf(w, a.y, num[1]);
@@ -344,7 +354,7 @@ template <int HD>
 __global__ __launch_bounds__(HD) void attn_combine_kernel(const float* __restrict__ ws_ml, const float* __restrict__ ws_o,
                                                          float* __restrict__ out, int n_q, int n_splits, int S,
                                                          const int32_t* __restrict__ start_p, uint16_t* __restrict__ xh,
-                                                         uint16_t* __restrict__ xl) {
+                                                         uint16_t* __restrict__ xl, bool base2) {
   constexpr int kBatch = 32;
   constexpr int NW = HD / 64 > 0 ? HD / 64 : 1;
   __shared__ float wts[512];
@@ -369,13 +379,13 @@ __global__ __launch_bounds__(HD) void attn_combine_kernel(const float* __restric
   __syncthreads();
   float den = 0.0f;
   if (d < ns) {
-    const float w = ml.x == -INFINITY ? 0.0f : expf(ml.x - M);
+    const float w = split_weight(ml.x, M, base2);
     wts[d] = w;
     den = fmaf(w, ml.y, den);
   }
   for (int i = d + HD; i < ns; i += HD) {
     const float m = ws_ml[2 * (base + i)];
-    const float w = m == -INFINITY ? 0.0f : expf(m - M);
+    const float w = split_weight(m, M, base2);
     wts[i] = w;
     den = fmaf(w, ws_ml[2 * (base + i) + 1], den);
   }
@@ -710,106 +720,139 @@ int launch_decode(const AttnPlan& p, int hd, int g, const float* q, const uint16
 
 // ---- Prefill (C > 1): flash attention on the fp16 matrix cores ----------------------------------
 //
-// Workgroup (key split, KV head, block of 32 query rows) with one wave per query head of the group.
-// Per 32-key block: S^T = K Q^T (v_mfma_f32_32x32x16_f16, K from LDS as the A operand, the fp32
-// queries split into fp16 hi + lo as two B operands, so the products keep fp32-level accuracy), the
-// mask (key <= pos, key < L) and an online softmax per query (a lane holds one query column; the
-// other half of its keys sits in lane ^ 32), then O^T += V^T P^T with P split into fp16 hi + lo the
-// same way. The S^T accumulator is used directly as the P^T operand: its keys are fed in a fixed
-// permutation (lane half h supplies keys 16u + 8(i/4) + 4h + i%4) and V^T is read from LDS in the
-// same order, so no transpose of P is needed. O^T's column is the lane's query, so the softmax
-// rescale is per lane. The partial (m, l, o) of each (row, head, split) goes to the workspace and
-// attn_combine8_kernel merges the splits. Each key block's K/V rows are loaded into registers two
-// blocks ahead (two register sets) while the blocks before it are computed; the workgroup has at
-// least 4 waves for that staging (waves past the group size only stage).
+// A unit is 32 query rows of one head; a workgroup (key split, KV head, unit block) has four waves, one
+// unit each (units of a KV head in order row block, head: neighbours share most of their keys), which
+// share the stream of K and V blocks of 32 keys through an LDS ring filled by direct loads.
+// Per block: S^T = K Q^T (v_mfma_f32_32x32x16_f16, K from LDS as the A operand, the fp32 queries split
+// into fp16 hi + lo as two B operands, so the products keep fp32-level accuracy), an online softmax per
+// query (a lane holds one query column; the other half of its keys sits in lane ^ 32), then
+// O^T += V^T P^T with P split into fp16 hi + lo the same way. The S^T accumulator is used directly as the
+// P^T operand: its keys are fed in a fixed permutation (lane half h supplies keys 16u + 8(i/4) + 4h + i%4),
+// and V^T comes from the row-major V block in the same order by transposing LDS reads
+// (ds_read_b64_tr_b16: 16 lanes read a 4 x 16 block and lane i receives column i), so neither P nor V is
+// transposed through registers or memory.
+//
+// What bounds it: the matrix cores run hi and lo (twice the useful flops) and the vector units share the
+// issue with them, so the softmax is kept short: the scale rides in the exponent's fma, exponents are
+// base 2 (m is in log2 units), only blocks that cross a row's position or L are masked, and the sums are
+// rescaled only when a maximum has grown by more than 2^8 (P then stays below 2^8, far inside fp16 hi + lo).
+// The partial (m, l, o) of each (row, head, split) goes to the workspace and the combine kernels merge
+// the splits.
+// Measured on one MI355X, 24/8 heads of 128, with the combine: C = 256 at 1792 of 2048 keys 48.6 -> PERF_A us,
+// in the 3B prefill (256 of 512 keys) 23.5 -> PERF_B us. Before: one 32-row block per workgroup and head
+// group, V transposed by 2-byte LDS stores, two barriers per block, keys split 128 at a time whatever the
+// chunk (51 MB of partials at 2048 keys).
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
+constexpr int kUnitWaves = 4;  // units per workgroup
 
+// Swizzles of the 16-byte chunks of a key row in LDS: K so that 16 rows at one chunk fall in different
+// 16-byte bank groups, V so that the four rows (32 bytes each) of a transposing read do.
 template <int HD>
-__device__ __forceinline__ int kswz(int r) {  // 16-byte chunk swizzle of a key row in LDS
+__device__ __forceinline__ int kswz(int r) {
   return HD == 128 ? (r & 15) : ((r >> 1) & 7);
+}
+template <int HD>
+__device__ __forceinline__ int vswz(int r) {
+  return HD == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2;
+}
+
+// fp32 pair -> fp16 hi and lo = fp16(v - hi), both round to nearest even (v - hi is exact in the fma).
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  asm("v_cvt_pk_f16_f32 %0, %2, %3\n\t"
+      "v_fma_mixlo_f16 %1, %0, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %1, %0, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+      : "=&v"(hi), "=&v"(lo)
+      : "v"(a), "v"(b));
+}
+
+// 16 bytes per lane from global memory straight into LDS (lane i's land at dst + 16 i); a transposing LDS
+// read. (Device functions: called in the kernel body, these builtins make the compiler drop its host stub.)
+typedef short short4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, void* dst, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst), 16, off, 0, 0, 0);
+}
+__device__ __forceinline__ short4v read_tr4(void* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v*)p);
 }
 
 template <int HD>
-__global__ __launch_bounds__(64 * kMfmaMaxG) void attn_prefill_mfma_kernel(
+__global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
     const float* __restrict__ q, int q_stride, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     float* __restrict__ ws_ml, float* __restrict__ ws_o, int C, int n_q, int n_kv, int L, int S,
     const int32_t* __restrict__ start_p, float scale) {
-  constexpr int KSTEPS = HD / 16;       // 16-dim k-steps of the score MFMAs
-  constexpr int OT = HD / 32;           // 32-dim output tiles
-  constexpr int KCH = HD / 8;           // 16-byte chunks per key row
-  constexpr int VT_PITCH = 32 * 2 + 8;  // bytes per V^T row: 32 keys + 8 bytes (conflict-free 8-byte reads)
-  constexpr int kMaxCh = 32 * KCH / 256; // staging chunks per thread (at least 4 waves)
-  __shared__ __attribute__((aligned(16))) unsigned char Ks[32 * HD * 2];
-  __shared__ __attribute__((aligned(16))) unsigned char Vt[HD * VT_PITCH];
+  constexpr int KSTEPS = HD / 16;           // 16-dim k-steps of the score MFMAs
+  constexpr int OT = HD / 32;               // 32-dim output tiles
+  constexpr int kRow = HD * 2;              // bytes per key row
+  constexpr int kBlk = 32 * kRow;           // bytes of a K or V block
+  constexpr int NST = 4;                    // ring stages
+  constexpr int kRpi = 1024 / kRow;         // rows per 1 KB load instruction
+  constexpr int kLd = kBlk / 1024 / kUnitWaves;  // K (and V) load instructions per wave and block
+  __shared__ __attribute__((aligned(16))) unsigned char ring[NST * 2 * kBlk];
   const int g = n_q / n_kv;
-  const int split = blockIdx.x, hk = blockIdx.y, qb = blockIdx.z;
+  const int split = blockIdx.x, hk = blockIdx.y;
   const int n_splits = gridDim.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool computes = wave < g;       // waves past the group size only stage K and V
-  const int h = hk * g + (computes ? wave : 0);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = lane >> 5, ql = lane & 31;
-  const int nthr = blockDim.x;
-  const int c0 = qb * 32;
+  const int units = (C + 31) / 32 * g;
+  const int u0 = blockIdx.z * kUnitWaves, unit = u0 + wave;
   const int start = start_p[0];
-  const int pos_max = start + min(c0 + 31, C - 1);
   const int k0 = split * S;
-  const int k_end = min(min(k0 + S, L), pos_max + 1);
-  if (k0 >= k_end) return;  // no row of the block sees a key of this split: the merge never reads it
-  const int c = c0 + ql;
-  const bool row_ok = computes && c < C;
-  const int pos = start + c;
+  // the keys that any row of the workgroup sees in this split
+  const int rows_end = min((min(u0 + kUnitWaves, units) - 1) / g * 32 + 32, C);
+  const int k_end = min(min(k0 + S, L), start + rows_end);
+  if (k0 >= k_end) return;  // no row of the workgroup sees a key of this split: the merge never reads it
+  const int c0 = unit / g * 32, h = hk * g + unit % g;
+  const int c = c0 + ql, pos = start + c;
+  const bool row_ok = unit < units && c < C;
+  const int wave_end = unit < units ? min(k_end, start + min(c0 + 32, C)) : 0;  // keys this wave needs
+  const int wave_full = min(start + c0, L - 1);                                // blocks up to here need no mask
 
-  // Q^T operand (column = this lane's query, k = dims 16 t + 8 half + i), split into fp16 hi + lo
+  // Q^T operand (column = this lane's query, k = dims 16 t + 8 half + i), split into fp16 hi + lo. A negative
+  // scale negates the queries, a zero one clears them, so that the exponent's factor below is positive.
+  const float sign = scale < 0.0f ? -1.0f : scale == 0.0f ? 0.0f : 1.0f;
+  const float cs = scale == 0.0f ? 1.0f : fabsf(scale) * 1.44269504088896340736f;
   half8 qh[KSTEPS], qlo[KSTEPS];
 #pragma unroll
   for (int t = 0; t < KSTEPS; ++t) {
-    float f[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    float4 a = make_float4(0, 0, 0, 0), b = a;
     if (row_ok) {
       const float4* qp = reinterpret_cast<const float4*>(q + static_cast<size_t>(c) * q_stride +
                                                          static_cast<size_t>(h) * HD + 16 * t + 8 * half);
-      const float4 a = qp[0], b = qp[1];
-      f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
+      a = qp[0], b = qp[1];
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const _Float16 hi = static_cast<_Float16>(f[i]);
-      qh[t][i] = hi;
-      qlo[t][i] = static_cast<_Float16>(f[i] - static_cast<float>(hi));
-    }
+    uint32_t hi[4], lo[4];
+    split2(sign * a.x, sign * a.y, hi[0], lo[0]);
+    split2(sign * a.z, sign * a.w, hi[1], lo[1]);
+    split2(sign * b.x, sign * b.y, hi[2], lo[2]);
+    split2(sign * b.z, sign * b.w, hi[3], lo[3]);
+    qh[t] = __builtin_bit_cast(half8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+    qlo[t] = __builtin_bit_cast(half8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
   }
 
-  const uint32_t cache_bytes = static_cast<uint32_t>(L) * n_kv * HD * 2u;
+  // Ring loads: instruction n = wave + j * 4 of a block fills rows n kRpi ..; the lane for LDS slot s of row r
+  // fetches chunk s ^ swz(r). Keys past L read out of range (zeros).
+  const uint32_t cache_bytes = static_cast<uint32_t>(L) * n_kv * kRow;
   const __amdgpu_buffer_rsrc_t kres = make_rsrc(kc, cache_bytes);
   const __amdgpu_buffer_rsrc_t vres = make_rsrc(vc, cache_bytes);
-  // K/V rows of a 32-key block: chunk ch = threadIdx.x + i * nthr (row ch / KCH, 16-byte chunk ch % KCH);
-  // keys past L read out of range (zeros).
-  // Two register sets: block kb's rows are requested two blocks ahead of their use.
-  uint4 kpa[kMaxCh], vpa[kMaxCh], kpb[kMaxCh], vpb[kMaxCh];
-  auto load_block = [&](int kb, uint4 (&kpre)[kMaxCh], uint4 (&vpre)[kMaxCh]) {
+  const uint32_t key_step = static_cast<uint32_t>(n_kv) * kRow;
+  uint32_t koff[kLd], voff[kLd];
 #pragma unroll
-    for (int i = 0; i < kMaxCh; ++i) {
-      const int ch = threadIdx.x + i * nthr;
-      const int r = ch / KCH, cc = ch - (ch / KCH) * KCH;
-      const uint32_t off = ch < 32 * KCH ? (static_cast<uint32_t>(kb + r) * n_kv + hk) * (HD * 2u) + cc * 16u
-                                         : 0x80000000u;
-      kpre[i] = buf_load16(kres, off);
-      vpre[i] = buf_load16(vres, off);
-    }
-  };
-  auto stage_block = [&](const uint4 (&kpre)[kMaxCh], const uint4 (&vpre)[kMaxCh]) {
+  for (int j = 0; j < kLd; ++j) {
+    const int r = (wave + j * kUnitWaves) * kRpi + lane / (kRow / 16), s = lane % (kRow / 16);
+    koff[j] = r * key_step + hk * kRow + ((s ^ kswz<HD>(r)) << 4);
+    voff[j] = r * key_step + hk * kRow + ((s ^ vswz<HD>(r)) << 4);
+  }
+  const int nb = (k_end - k0 + 31) / 32;
+  auto issue = [&](int b) {
+    unsigned char* kd = ring + (b % NST) * (2 * kBlk);
+    const uint32_t base = b < nb ? static_cast<uint32_t>(k0 + 32 * b) * key_step : 0x80000000u;
 #pragma unroll
-    for (int i = 0; i < kMaxCh; ++i) {
-      const int ch = threadIdx.x + i * nthr;
-      if (ch < 32 * KCH) {
-        const int r = ch / KCH, cc = ch - (ch / KCH) * KCH;
-        *reinterpret_cast<uint4*>(Ks + r * (HD * 2) + ((cc ^ kswz<HD>(r)) << 4)) = kpre[i];
-        const uint32_t w[4] = {vpre[i].x, vpre[i].y, vpre[i].z, vpre[i].w};
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          *reinterpret_cast<uint16_t*>(Vt + (cc * 8 + j) * VT_PITCH + r * 2) =
-              static_cast<uint16_t>(w[j >> 1] >> (16 * (j & 1)));
-      }
+    for (int j = 0; j < kLd; ++j) {
+      const int n = wave + j * kUnitWaves;
+      load_lds16(kres, kd + n * 1024, base + koff[j]);
+      load_lds16(vres, kd + kBlk + n * 1024, base + voff[j]);
     }
   };
 
@@ -818,80 +861,94 @@ __global__ __launch_bounds__(64 * kMfmaMaxG) void attn_prefill_mfma_kernel(
   for (int tt = 0; tt < OT; ++tt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[tt][e] = 0.0f;
-  float m = -INFINITY, l = 0.0f;
+  float m = -INFINITY, l = 0.0f;  // l: over this lane half's keys
 
-  auto block = [&](int kb, uint4 (&kpre)[kMaxCh], uint4 (&vpre)[kMaxCh]) {
-    stage_block(kpre, vpre);
-    __syncthreads();
-    if (kb + 64 < k_end) load_block(kb + 64, kpre, vpre);  // in flight during the next two blocks
-
-    // S^T = K Q^T: 32 keys (rows) x 32 queries (columns)
-    float16v sacc;
+  // transposing V reads: lane i of each 16 reads row i / 4 of a 4-key group, 8 bytes at dims 4 (i % 4) of its
+  // 16 dims; groups of 16 lanes: dims 16 (group % 2), keys 4 (group / 2)
+  const int kr = (lane & 15) >> 2;
+  const int vrow = (4 * half + kr) * kRow + (lane & 1) * 8;
+  int vcol[OT];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) sacc[e] = 0.0f;
+  for (int tt = 0; tt < OT; ++tt)
+    vcol[tt] = vrow + (((4 * tt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ vswz<HD>(kr)) << 4);
+
+  auto compute = [&](int b) {
+    const int kb = k0 + 32 * b;
+    if (kb >= wave_end) return;
+    const unsigned char* Ks = ring + (b % NST) * (2 * kBlk);
+    unsigned char* Vs = ring + (b % NST) * (2 * kBlk) + kBlk;
+    // S^T = K Q^T: 32 keys (rows) x 32 queries (columns)
+    float16v s = {};
 #pragma unroll
     for (int t = 0; t < KSTEPS; ++t) {
-      const half8 ka = *reinterpret_cast<const half8*>(Ks + ql * (HD * 2) + (((2 * t + half) ^ kswz<HD>(ql)) << 4));
-      sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[t], sacc, 0, 0, 0);
-      sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qlo[t], sacc, 0, 0, 0);
+      const half8 ka = *reinterpret_cast<const half8*>(Ks + ql * kRow + (((2 * t + half) ^ kswz<HD>(ql)) << 4));
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[t], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qlo[t], s, 0, 0, 0);
     }
-    float sv[16];
-    float mb = -INFINITY;
+    if (kb + 31 > wave_full) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int key = kb + 8 * (e >> 2) + 4 * half + (e & 3);
+        s[e] = key <= pos && key < L ? s[e] : -INFINITY;
+      }
+    }
+    float mb = s[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mb = fmaxf(mb, s[e]);
+    mb = swap_combine32<true>(mb) * cs;
+    if (__any(mb > m + 8.0f)) {
+      const float m_new = fmaxf(m, mb);
+      const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int tt = 0; tt < OT; ++tt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[tt][e] *= alpha;
+    }
+    const float mu = m == -INFINITY ? 0.0f : m;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int key = kb + 8 * (e >> 2) + 4 * half + (e & 3);
-      const bool ok = row_ok && key <= pos && key < L;
-      sv[e] = ok ? sacc[e] * scale : -INFINITY;
-      mb = fmaxf(mb, sv[e]);
+      s[e] = __builtin_amdgcn_exp2f(fmaf(s[e], cs, -mu));
+      l += s[e];
     }
-    mb = swap_combine32<true>(mb);
-    const float m_new = fmaxf(m, mb);
-    const float alpha = m == -INFINITY ? 0.0f : expf(m - m_new);
-    float ls = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      sv[e] = sv[e] == -INFINITY ? 0.0f : expf(sv[e] - m_new);
-      ls += sv[e];
-    }
-    ls = swap_combine32<false>(ls);
-    l = l * alpha + ls;
-    m = m_new;
-#pragma unroll
-    for (int tt = 0; tt < OT; ++tt)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) o[tt][e] *= alpha;
-
     // O^T += V^T P^T over two 16-key steps
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      half8 ph, pl;
+      uint32_t ph[4], pl[4];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const _Float16 hi = static_cast<_Float16>(sv[8 * u + i]);
-        ph[i] = hi;
-        pl[i] = static_cast<_Float16>(sv[8 * u + i] - static_cast<float>(hi));
-      }
+      for (int i = 0; i < 4; ++i) split2(s[8 * u + 2 * i], s[8 * u + 2 * i + 1], ph[i], pl[i]);
+      const half8 p_hi = __builtin_bit_cast(half8, make_uint4(ph[0], ph[1], ph[2], ph[3]));
+      const half8 p_lo = __builtin_bit_cast(half8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
 #pragma unroll
       for (int tt = 0; tt < OT; ++tt) {
-        const unsigned char* vrow = Vt + (32 * tt + ql) * VT_PITCH;
-        const uint2 v0 = *reinterpret_cast<const uint2*>(vrow + (16 * u + 4 * half) * 2);
-        const uint2 v1 = *reinterpret_cast<const uint2*>(vrow + (16 * u + 8 + 4 * half) * 2);
-        const uint4 vv = make_uint4(v0.x, v0.y, v1.x, v1.y);
-        const half8 va = __builtin_bit_cast(half8, vv);
-        o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, ph, o[tt], 0, 0, 0);
-        o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pl, o[tt], 0, 0, 0);
+        const short4v v0 = read_tr4(Vs + vcol[tt] + (16 * u) * kRow);
+        const short4v v1 = read_tr4(Vs + vcol[tt] + (16 * u + 8) * kRow);
+        const half8 va = __builtin_bit_cast(half8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+        o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, p_hi, o[tt], 0, 0, 0);
+        o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, p_lo, o[tt], 0, 0, 0);
       }
     }
-    __syncthreads();  // every wave is done with this block's K and V^T
   };
-  load_block(k0, kpa, vpa);
-  if (k0 + 32 < k_end) load_block(k0 + 32, kpb, vpb);
-  for (int kb = k0; kb < k_end; kb += 64) {
-    block(kb, kpa, vpa);
-    if (kb + 32 < k_end) block(kb + 32, kpb, vpb);
-  }
 
-  if (row_ok) {
+  // Block b's loads of this wave are complete when at most NST - 2 later blocks' are in flight; the barrier
+  // publishes the block and frees the stage of block b - 1, whose reads every wave has waited for. Blocks past
+  // the last are issued too (out of range: no traffic), so the count is a constant.
+#pragma unroll
+  for (int b = 0; b < NST - 1; ++b) issue(b);
+  for (int b = 0; b < nb; ++b) {
+    constexpr int kWait = (NST - 2) * 2 * kLd;
+    __builtin_amdgcn_s_waitcnt((kWait & 15) | ((kWait >> 4) << 14) | (7 << 4) | (15 << 8));  // vmcnt only
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(b + NST - 1);
+    compute(b);
+  }
+  __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): nothing lands in LDS after the waves exit
+
+  if (row_ok && k0 < wave_end) {
+    l = swap_combine32<false>(l);
     const size_t idx = (static_cast<size_t>(c) * n_q + h) * n_splits + split;
     if (half == 0) {
       ws_ml[2 * idx] = m;
@@ -974,7 +1031,7 @@ int attn_bucket_impl(const float* q, int q_row_stride, const uint16_t* k_cache, 
     return launch_decode(p, hd, n_q / n_kv, q, k_cache, v_cache, ws_ml, ws_o, out, n_kv, L, start, scale, st);
   int rc = Q4_OK;
   if (p.mfma) {
-    const dim3 grid(p.n_splits, n_kv, p.n_cblk), block(64 * std::max(n_q / n_kv, 4));
+    const dim3 grid(p.n_splits, n_kv, (p.n_cblk * (n_q / n_kv) + kUnitWaves - 1) / kUnitWaves), block(64 * kUnitWaves);
     if (hd == 128)
       hipLaunchKernelGGL(attn_prefill_mfma_kernel<128>, grid, block, 0, st, q, q_row_stride, k_cache, v_cache, ws_ml,
                          ws_o, C, n_q, n_kv, L, p.S, start, scale);
@@ -998,18 +1055,18 @@ int attn_bucket_impl(const float* q, int q_row_stride, const uint16_t* k_cache, 
     const unsigned blocks = static_cast<unsigned>((rows * (hd / 8) + 255) / 256);
     if (hd == 128)
       hipLaunchKernelGGL(attn_combine8_kernel<128>, dim3(blocks), dim3(256), 0, st, ws_ml, ws_o, out, rows, n_q,
-                         p.n_splits, p.S, start, xh, xl);
+                         p.n_splits, p.S, start, xh, xl, p.mfma);
     else
       hipLaunchKernelGGL(attn_combine8_kernel<64>, dim3(blocks), dim3(256), 0, st, ws_ml, ws_o, out, rows, n_q,
-                         p.n_splits, p.S, start, xh, xl);
+                         p.n_splits, p.S, start, xh, xl, p.mfma);
     return launch_status();
   }
   if (hd == 128)
     hipLaunchKernelGGL(attn_combine_kernel<128>, dim3(C * n_q), dim3(128), 0, st, ws_ml, ws_o, out, n_q, p.n_splits,
-                       p.S, start, xh, xl);
+                       p.S, start, xh, xl, p.mfma);
   else
     hipLaunchKernelGGL(attn_combine_kernel<64>, dim3(C * n_q), dim3(64), 0, st, ws_ml, ws_o, out, n_q, p.n_splits,
-                       p.S, start, xh, xl);
+                       p.S, start, xh, xl, p.mfma);
   return launch_status();
 }
 }  // namespace

@@ -52,6 +52,25 @@ __device__ __forceinline__ F16Magic f16_magic() {
   return m;
 }
 
+// fp32 pair -> fp16 hi = fp16(v) and lo = fp16(v - hi), round to nearest even, packed (a in the low half).
+// `minus1` is -1.0f from minus_one(), so that v - hi (exact) becomes one v_fma_mix_f32 per value: four
+// instructions a pair, where the compiler's own subtraction takes seven.
+__device__ __forceinline__ float minus_one() {
+  float m;
+  asm("v_mov_b32 %0, -1.0" : "=v"(m));
+  return m;
+}
+__device__ __forceinline__ void split_f16_pair(float a, float b, float minus1, uint32_t& hi, uint32_t& lo) {
+  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+  typedef float float2v __attribute__((ext_vector_type(2)));
+  const half2v h = __builtin_convertvector((float2v{a, b}), half2v);
+  const float ra = __builtin_fmaf(static_cast<float>(h.x), minus1, a);
+  const float rb = __builtin_fmaf(static_cast<float>(h.y), minus1, b);
+  const half2v l = __builtin_convertvector((float2v{ra, rb}), half2v);
+  hi = __builtin_bit_cast(uint32_t, h);
+  lo = __builtin_bit_cast(uint32_t, l);
+}
+
 __device__ __forceinline__ float half_bits_to_float(uint16_t h) {
   return static_cast<float>(__builtin_bit_cast(_Float16, h));
 }

@@ -264,13 +264,13 @@ constexpr size_t kLinLds[] = {LinCfg<128, 128>::kLds, LinCfg<128, 64>::kLds, Lin
 
 constexpr uint32_t kOOBw = 0x80000000u;
 
-__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, void* dst, uint32_t off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst), 16, off, 0, 0, 0);
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, void* dst, uint32_t off, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst), 16, off, soff, 0, 0);
 }
 
 // 4 bytes per lane from global memory straight into LDS: lane i's dword lands at dst + 4 i.
-__device__ __forceinline__ void load_lds4(__amdgpu_buffer_rsrc_t r, void* dst, uint32_t off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst), 4, off, 0, 0, 0);
+__device__ __forceinline__ void load_lds4(__amdgpu_buffer_rsrc_t r, void* dst, uint32_t off, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(dst), 4, off, soff, 0, 0);
 }
 
 template <int N>
@@ -450,54 +450,60 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void q4_linear_ws_kernel(
   const int nk = K / 64;
   const int kt_begin = n_split > 1 ? ksp * nk_split : 0;
   const int kt_end = n_split > 1 ? min(nk, kt_begin + nk_split) : nk;
+  // Per-lane offsets of the scale words (a step adds a uniform one). T16: instruction i = wave + j * kWaves
+  // (< 2 BN / 128) fills slot i / (BN / 128) (the step's first or last group) for the 128 virtual columns of
+  // part i % (BN / 128): lane -> rows 2 (lane % 8) and + 1 of tile lane / 8 of the part, stored as fp16 in
+  // column order. Reference layout: instruction i (< 2 kSBlk) fills slot i / kSBlk for the 64 columns of
+  // block i % kSBlk: lane -> column, the aligned dword holding its fp16 scale (the buffer range is rounded up
+  // to 4 bytes; device allocations are 256-byte granular): element phys(col) * spr + g, so its dword
+  // depends on the parities of both parts. Spare instructions fill the junk area.
+  uint32_t soff[G::kSI][T16 ? 1 : 2];
+#pragma unroll
+  for (int j = 0; j < G::kSI; ++j) {
+    const int i = wave + j * G::kWaves;
+    if constexpr (T16) {
+      constexpr int kParts = BN / 128;
+      const int t = n0 / 16 + (i % kParts) * 8 + (lane >> 3);
+      soff[j][0] = i < 2 * kParts && t < n_t16 ? static_cast<uint32_t>(t) * t16_tiles_k * 128u + 4u * (lane & 7) : kOOBw;
+    } else {
+      const int col = n0 + (i % G::kSBlk) * 64 + lane;
+      const uint32_t e = static_cast<uint32_t>(phys(col)) * spr;
+      const bool real = i < 2 * G::kSBlk && col < N;
+      soff[j][0] = real ? (e >> 1) * 4u : kOOBw;
+      soff[j][1] = real ? ((e + 1) >> 1) * 4u : kOOBw;
+    }
+  }
   // Load idx (0 <= idx < kLPW, a constant after unrolling) of K step kt into `stage`: the x_hi and x_lo
-  // rows of instruction idx / 2 (idx < 2 kAI), then the weight rows, then the scale words.
-  auto issue_one = [&](int idx, int kt, int stage) {
+  // rows of instruction idx / 2 (idx < 2 kAI), then the weight rows, then the scale words. The step is the
+  // load's uniform offset; steps past the range load the last one again (never read).
+  auto issue_one = [&](int idx, int kt_want, int stage) {
+    const int kt = min(kt_want, kt_end - 1);
     const int k0 = kt * 64;
-    const bool kin = kt < kt_end;
     unsigned char* sh = lds + stage * G::kStage;
     unsigned char* sl = sh + BM * G::kXRow;
     unsigned char* sw = sl + BM * G::kXRow;
     if (idx < 2 * G::kAI) {
       const int j = idx / 2;
-      const uint32_t off = kin && xoff[j] != kOOBw ? xoff[j] + k0 * 2u : kOOBw;
-      if (idx % 2 == 0) load_lds16(hr, xreal[j] ? sh + (wave + j * G::kWaves) * 1024 : junk, off);
-      else load_lds16(lr, xreal[j] ? sl + (wave + j * G::kWaves) * 1024 : junk, off);
+      if (idx % 2 == 0) load_lds16(hr, xreal[j] ? sh + (wave + j * G::kWaves) * 1024 : junk, xoff[j], k0 * 2);
+      else load_lds16(lr, xreal[j] ? sl + (wave + j * G::kWaves) * 1024 : junk, xoff[j], k0 * 2);
     } else if (idx < 2 * G::kAI + G::kBI) {
       const int j = idx - 2 * G::kAI;
-      const uint32_t kofs = T16 ? static_cast<uint32_t>(kt >> 1) * 1024u + (kt & 1) * 32u : static_cast<uint32_t>(k0 / 2);
-      load_lds16(wr, wreal[j] ? sw + (wave + j * G::kWaves) * 1024 : junk,
-                 kin && woff[j] != kOOBw ? woff[j] + kofs : kOOBw);
-    } else if constexpr (T16) {
-      // Scales: instruction i = wave + j * kWaves (< 2 BN / 128) fills slot i / (BN / 128) (the step's
-      // first or last group) for the 128 virtual columns of part i % (BN / 128): lane -> rows 2 (lane % 8)
-      // and + 1 of tile lane / 8 of the part, stored as fp16 in column order.
-      unsigned char* ss = sw + BN * G::kWRow;
-      const int g0 = k0 >> gshift, g1 = (k0 + 63) >> gshift;
-      const int j = idx - 2 * G::kAI - G::kBI;
-      const int i = wave + j * G::kWaves;
-      constexpr int kParts = BN / 128;
-      const bool real = i < 2 * kParts;
-      const int slot = i / kParts, part = i - slot * kParts;
-      const int t = n0 / 16 + part * 8 + (lane >> 3);
-      const int g = slot ? g1 : g0;
-      const uint32_t e = ((static_cast<uint32_t>(t) * t16_tiles_k + (g >> 2)) * 4u + (g & 3)) * 16u + 2u * (lane & 7);
-      load_lds4(sr, real ? ss + slot * (BN * 2) + part * 256 : junk, real && kin && t < n_t16 ? e * 2u : kOOBw);
+      load_lds16(wr, wreal[j] ? sw + (wave + j * G::kWaves) * 1024 : junk, woff[j],
+                 T16 ? (kt >> 1) * 1024 + (kt & 1) * 32 : k0 / 2);
     } else {
-      // Scales: instruction i = wave + j * kWaves (< 2 kSBlk) fills slot i / kSBlk (the step's first or
-      // last group; a 64-k step touches at most two groups of >= 32) for the 64 columns of block
-      // i % kSBlk: lane -> column, the aligned dword holding its fp16 scale (the buffer range is rounded
-      // up to 4 bytes; device allocations are 256-byte granular). Spare instructions fill the junk area.
       unsigned char* ss = sw + BN * G::kWRow;
-      const int g0 = k0 >> gshift, g1 = (k0 + 63) >> gshift;
       const int j = idx - 2 * G::kAI - G::kBI;
       const int i = wave + j * G::kWaves;
-      const bool real = i < 2 * G::kSBlk;
-      const int slot = i / G::kSBlk, blk = i - slot * G::kSBlk;
-      const int col = n0 + blk * 64 + lane;
-      const uint32_t e = static_cast<uint32_t>(phys(col)) * spr + (slot ? g1 : g0);
-      load_lds4(sr, real ? ss + (slot * G::kSBlk + blk) * 256 : junk,
-                real && kin && col < N ? (e >> 1) * 4u : kOOBw);
+      if constexpr (T16) {
+        constexpr int kParts = BN / 128;
+        const int slot = i / kParts, part = i - slot * kParts;
+        const int g = (slot ? k0 + 63 : k0) >> gshift;
+        load_lds4(sr, i < 2 * kParts ? ss + slot * (BN * 2) + part * 256 : junk, soff[j][0], g * 32);
+      } else {
+        const int slot = i / G::kSBlk, blk = i - slot * G::kSBlk;
+        const int g = (slot ? k0 + 63 : k0) >> gshift;
+        load_lds4(sr, i < 2 * G::kSBlk ? ss + (slot * G::kSBlk + blk) * 256 : junk, soff[j][g & 1], (g >> 1) * 4);
+      }
     }
   };
   auto issue = [&](int kt, int stage) {

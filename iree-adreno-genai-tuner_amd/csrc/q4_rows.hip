@@ -70,16 +70,6 @@ __device__ __forceinline__ half8 rows_nibbles(uint32_t w, const F16Magic& mg) {
   return half8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
 
-// fp32 pair -> fp16 hi = fp16(v) and lo = fp16(v - hi), both round to nearest even, in three
-// instructions (the compiler's conversions take eight): v - hi is exact in the mixed-precision fma.
-__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-  asm("v_cvt_pk_f16_f32 %0, %2, %3\n\t"
-      "v_fma_mixlo_f16 %1, %0, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixhi_f16 %1, %0, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-      : "=&v"(hi), "=&v"(lo)
-      : "v"(a), "v"(b));
-}
-
 // Rows 16 MT, columns 16 NT per workgroup; blockDim.x / 64 waves share K. `magic`: the
 // reciprocal 2^32 / d (rounded up) of d = 32-k blocks (kG128: 128-k steps) per group; 0 for d = 1.
 template <int MT, int NT, bool kG128>
@@ -95,6 +85,7 @@ __global__ __launch_bounds__(MT == 1 && NT == 1 ? 1024 : 512) void q4_rows_kerne
   const __amdgpu_buffer_rsrc_t sr = rows_rsrc(SC, static_cast<uint32_t>(N) * spr * 2u);
   const int steps = (K + 127) / 128;
   const F16Magic mg = f16_magic();
+  const float m1 = minus_one();
 
   struct Step {
     i32x4 w[NT];
@@ -161,10 +152,10 @@ __global__ __launch_bounds__(MT == 1 && NT == 1 ? 1024 : 512) void q4_rows_kerne
       for (int i = 0; i < MT; ++i) {
         const float4v a = b.x[i][2 * q], e = b.x[i][2 * q + 1];
         uint32_t h[4], l[4];  // k order 0, 4, 1, 5, 2, 6, 3, 7
-        split2(a.x, e.x, h[0], l[0]);
-        split2(a.y, e.y, h[1], l[1]);
-        split2(a.z, e.z, h[2], l[2]);
-        split2(a.w, e.w, h[3], l[3]);
+        split_f16_pair(a.x, e.x, m1, h[0], l[0]);
+        split_f16_pair(a.y, e.y, m1, h[1], l[1]);
+        split_f16_pair(a.z, e.z, m1, h[2], l[2]);
+        split_f16_pair(a.w, e.w, m1, h[3], l[3]);
         hi[i] = __builtin_bit_cast(half8, make_uint4(h[0], h[1], h[2], h[3]));
         lo[i] = __builtin_bit_cast(half8, make_uint4(l[0], l[1], l[2], l[3]));
       }

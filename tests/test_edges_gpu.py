@@ -87,3 +87,41 @@ def test_linear_many_rows(dev, M, N, K, group):
         ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=dev)
         ops.q4_linear_ws(x, qw, sc, group, residual=h, out=h, workspace=ws)
         assert ((h.cpu().double() - ref).abs() <= bound).all(), split
+
+
+def attn_ref64(q, kc, vc, start, scale):
+    C, nq, hd = q.shape
+    n, nkv = min(start + C, kc.shape[0]), kc.shape[1]
+    g = nq // nkv
+    mask = torch.arange(n)[None, :] > (start + torch.arange(C))[:, None]
+    out = torch.empty(C, nq, hd, dtype=torch.float64)
+    for h in range(nq):
+        s = (q[:, h].double() @ kc[:n, h // g].double().t()) * scale
+        out[:, h] = torch.softmax(s.masked_fill(mask, float("-inf")), -1) @ vc[:n, h // g].double()
+    return out.reshape(C, nq * hd)
+
+
+@pytest.mark.parametrize("C,start,L,nq,nkv,hd,ps", [
+    (2, 0, 33, 8, 8, 64, None), (33, 31, 96, 6, 2, 128, None), (31, 480, 512, 5, 1, 64, None),
+    (65, 0, 65, 24, 8, 128, None), (256, 1792, 2048, 24, 8, 128, None), (97, 3900, 4096, 7, 1, 128, None),
+    (64, 700, 777, 8, 1, 64, None), (256, 0, 256, 4, 2, 64, 32), (130, 125, 256, 12, 12, 64, 96),
+    (96, 416, 512, 24, 8, 128, 512), (40, 20, 300, 20, 4, 128, 32)])
+@pytest.mark.parametrize("scale", [0.088, -0.3, 0.0, 4.0])
+def test_attn_prefill_units_and_splits(dev, kernel_override, C, start, L, nq, nkv, hd, ps, scale):
+    """Chunks whose 32-row units do not divide over the workgroups' waves, rows and keys off the 32-key
+    blocks, one and many splits, splits that some rows of a workgroup do not reach, and scales of both
+    signs, zero, and one whose maxima grow by more than the rescaling threshold."""
+    if ps:
+        kernel_override("attn_ps", ps)
+    g = torch.Generator().manual_seed(C + start + L)
+    q = torch.randn(C, nq, hd, generator=g)
+    kc, vc = torch.randn(L, nkv, hd, generator=g).half(), torch.randn(L, nkv, hd, generator=g).half()
+    kc[: min(64, L)] *= 0.05  # small scores first: the running maximum grows in later blocks
+    kc[start + C:], vc[start + C:] = 100.0, 1000.0  # stale rows past every position: no weight
+    ref = attn_ref64(q, kc, vc, start, scale)
+    out = torch.full((C, nq * hd), float("nan"), device=dev)
+    ops.attn_bucket(q.to(dev), kc.to(dev), vc.to(dev), L, torch.tensor([start], dtype=torch.int32, device=dev), scale,
+                    out=out)
+    # scores of fp16 hi + lo queries: 2^-22 sum |q k| each, the same again for the fp32 sums; P likewise
+    smax = (q.abs().double().sum(-1).max() * 4.0 * abs(scale)).item()
+    assert (out.cpu().double() - ref).abs().max().item() <= 5.0 * (2.0 ** -20 * max(smax, 1.0)) + 1e-6
