@@ -47,12 +47,12 @@ AttnPlan plan_for(int C, int n_q, int n_kv, int L) {
     const int ov = debug_override(Q4_DBG_ATTN_S);  // sweep override: keys per split (32, 64 or 128)
     if (ov == 32 || ov == 64 || ov == 128) p.S = ov;
   } else if (g <= kMfmaMaxG && !debug_flag(Q4_DBG_ATTN_GENERIC)) {
-    // Keys per split: enough for about two workgroups of four 32-row units per CU, at least 64 (128 past
+    // Keys per split: enough for about one workgroup of four 32-row units per CU, at least 64 (128 past
     // 256 keys): more splits only add partials to write and merge.
     p.mfma = true;
     p.CB = 32;
     const int64_t wgs = static_cast<int64_t>(n_kv) * (((C + 31) / 32 * g + 3) / 4);  // per split
-    const int64_t want = std::max<int64_t>(1, 512 / wgs);
+    const int64_t want = std::max<int64_t>(1, 256 / wgs);
     p.S = std::max(L <= 256 ? 64 : 128, static_cast<int>((L + 32 * want - 1) / (32 * want)) * 32);
     const int ov = debug_override(Q4_DBG_ATTN_PS);  // sweep override: keys per split (a multiple of 32, <= 512)
     if (ov != Q4_DBG_UNSET && ov >= 32 && ov <= 512 && ov % 32 == 0) p.S = ov;
@@ -738,13 +738,17 @@ int launch_decode(const AttnPlan& p, int hd, int g, const float* q, const uint16
 // rescaled only when a maximum has grown by more than 2^8 (P then stays below 2^8, far inside fp16 hi + lo).
 // The partial (m, l, o) of each (row, head, split) goes to the workspace and the combine kernels merge
 // the splits.
-// Measured on one MI355X, 24/8 heads of 128, with the combine: C = 256 at 1792 of 2048 keys 48.6 -> PERF_A us,
-// in the 3B prefill (256 of 512 keys) 23.5 -> PERF_B us. Before: one 32-row block per workgroup and head
-// group, V transposed by 2-byte LDS stores, two barriers per block, keys split 128 at a time whatever the
-// chunk (51 MB of partials at 2048 keys).
+// Measured on one MI355X, 24/8 heads of 128, the combine included (us): C = 256 of 2048 keys 48.6 -> 30.0, of
+// 4096 91.8 -> 41, of 512 23.5 -> 19.7; 12/12 heads of 64, 256 of 2048 keys 16.7. Before: one 32-row block
+// and head group per workgroup, V transposed by 2-byte LDS stores, two barriers a block, a mask, an expf and a
+// rescaling on every block, and keys split 128 at a time whatever the chunk (51 MB of partials at 2048
+// keys). Of the 12.8 us of the kernel at 512 keys, writing the partials takes 4.4, the blocks 6.2, the
+// queries 2.2. Two waves per unit (even and odd blocks, merged through LDS) gave 5% at 2048 keys and more
+// and cost 10% below.
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
-constexpr int kUnitWaves = 4;  // units per workgroup
+constexpr int kUnits = 4;       // units, and waves, per workgroup
+constexpr int kRingStages = 4;  // one K and one V block each
 
 // Swizzles of the 16-byte chunks of a key row in LDS: K so that 16 rows at one chunk fall in different
 // 16-byte bank groups, V so that the four rows (32 bytes each) of a transposing read do.
@@ -755,15 +759,6 @@ __device__ __forceinline__ int kswz(int r) {
 template <int HD>
 __device__ __forceinline__ int vswz(int r) {
   return HD == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2;
-}
-
-// fp32 pair -> fp16 hi and lo = fp16(v - hi), both round to nearest even (v - hi is exact in the fma).
-__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-  asm("v_cvt_pk_f16_f32 %0, %2, %3\n\t"
-      "v_fma_mixlo_f16 %1, %0, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixhi_f16 %1, %0, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-      : "=&v"(hi), "=&v"(lo)
-      : "v"(a), "v"(b));
 }
 
 // 16 bytes per lane from global memory straight into LDS (lane i's land at dst + 16 i); a transposing LDS
@@ -777,17 +772,18 @@ __device__ __forceinline__ short4v read_tr4(void* p) {
 }
 
 template <int HD>
-__global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
+__global__ __launch_bounds__(64 * kUnits, 2) void attn_prefill_mfma_kernel(
     const float* __restrict__ q, int q_stride, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     float* __restrict__ ws_ml, float* __restrict__ ws_o, int C, int n_q, int n_kv, int L, int S,
-    const int32_t* __restrict__ start_p, float scale) {
+    const int32_t* __restrict__ start_p, float scale, float* __restrict__ out, uint16_t* __restrict__ xh,
+    uint16_t* __restrict__ xl) {
   constexpr int KSTEPS = HD / 16;           // 16-dim k-steps of the score MFMAs
   constexpr int OT = HD / 32;               // 32-dim output tiles
   constexpr int kRow = HD * 2;              // bytes per key row
   constexpr int kBlk = 32 * kRow;           // bytes of a K or V block
-  constexpr int NST = 4;                    // ring stages
+  constexpr int NST = kRingStages;
   constexpr int kRpi = 1024 / kRow;         // rows per 1 KB load instruction
-  constexpr int kLd = kBlk / 1024 / kUnitWaves;  // K (and V) load instructions per wave and block
+  constexpr int kLd = kBlk / 1024 / kUnits;  // K (and V) load instructions per wave and stage
   __shared__ __attribute__((aligned(16))) unsigned char ring[NST * 2 * kBlk];
   const int g = n_q / n_kv;
   const int split = blockIdx.x, hk = blockIdx.y;
@@ -796,11 +792,11 @@ __global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = lane >> 5, ql = lane & 31;
   const int units = (C + 31) / 32 * g;
-  const int u0 = blockIdx.z * kUnitWaves, unit = u0 + wave;
+  const int u0 = blockIdx.z * kUnits, unit = u0 + wave;
   const int start = start_p[0];
   const int k0 = split * S;
   // the keys that any row of the workgroup sees in this split
-  const int rows_end = min((min(u0 + kUnitWaves, units) - 1) / g * 32 + 32, C);
+  const int rows_end = min((min(u0 + kUnits, units) - 1) / g * 32 + 32, C);
   const int k_end = min(min(k0 + S, L), start + rows_end);
   if (k0 >= k_end) return;  // no row of the workgroup sees a key of this split: the merge never reads it
   const int c0 = unit / g * 32, h = hk * g + unit % g;
@@ -813,6 +809,7 @@ __global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
   // scale negates the queries, a zero one clears them, so that the exponent's factor below is positive.
   const float sign = scale < 0.0f ? -1.0f : scale == 0.0f ? 0.0f : 1.0f;
   const float cs = scale == 0.0f ? 1.0f : fabsf(scale) * 1.44269504088896340736f;
+  const float neg1 = minus_one();
   half8 qh[KSTEPS], qlo[KSTEPS];
 #pragma unroll
   for (int t = 0; t < KSTEPS; ++t) {
@@ -823,16 +820,16 @@ __global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
       a = qp[0], b = qp[1];
     }
     uint32_t hi[4], lo[4];
-    split2(sign * a.x, sign * a.y, hi[0], lo[0]);
-    split2(sign * a.z, sign * a.w, hi[1], lo[1]);
-    split2(sign * b.x, sign * b.y, hi[2], lo[2]);
-    split2(sign * b.z, sign * b.w, hi[3], lo[3]);
+    split_f16_pair(sign * a.x, sign * a.y, neg1, hi[0], lo[0]);
+    split_f16_pair(sign * a.z, sign * a.w, neg1, hi[1], lo[1]);
+    split_f16_pair(sign * b.x, sign * b.y, neg1, hi[2], lo[2]);
+    split_f16_pair(sign * b.z, sign * b.w, neg1, hi[3], lo[3]);
     qh[t] = __builtin_bit_cast(half8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
     qlo[t] = __builtin_bit_cast(half8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
   }
 
-  // Ring loads: instruction n = wave + j * 4 of a block fills rows n kRpi ..; the lane for LDS slot s of row r
-  // fetches chunk s ^ swz(r). Keys past L read out of range (zeros).
+  // Ring loads: instruction n = wave + j * kUnits of a block fills rows n kRpi ..; the lane for LDS slot
+  // s of row r fetches chunk s ^ swz(r). Keys past L read out of range (zeros).
   const uint32_t cache_bytes = static_cast<uint32_t>(L) * n_kv * kRow;
   const __amdgpu_buffer_rsrc_t kres = make_rsrc(kc, cache_bytes);
   const __amdgpu_buffer_rsrc_t vres = make_rsrc(vc, cache_bytes);
@@ -840,7 +837,7 @@ __global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
   uint32_t koff[kLd], voff[kLd];
 #pragma unroll
   for (int j = 0; j < kLd; ++j) {
-    const int r = (wave + j * kUnitWaves) * kRpi + lane / (kRow / 16), s = lane % (kRow / 16);
+    const int r = (wave + j * kUnits) * kRpi + lane / (kRow / 16), s = lane % (kRow / 16);
     koff[j] = r * key_step + hk * kRow + ((s ^ kswz<HD>(r)) << 4);
     voff[j] = r * key_step + hk * kRow + ((s ^ vswz<HD>(r)) << 4);
   }
@@ -850,7 +847,7 @@ __global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
     const uint32_t base = b < nb ? static_cast<uint32_t>(k0 + 32 * b) * key_step : 0x80000000u;
 #pragma unroll
     for (int j = 0; j < kLd; ++j) {
-      const int n = wave + j * kUnitWaves;
+      const int n = wave + j * kUnits;
       load_lds16(kres, kd + n * 1024, base + koff[j]);
       load_lds16(vres, kd + kBlk + n * 1024, base + voff[j]);
     }
@@ -878,13 +875,16 @@ __global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
     const unsigned char* Ks = ring + (b % NST) * (2 * kBlk);
     unsigned char* Vs = ring + (b % NST) * (2 * kBlk) + kBlk;
     // S^T = K Q^T: 32 keys (rows) x 32 queries (columns)
-    float16v s = {};
+    // (two accumulators: consecutive MFMAs do not wait for each other)
+    float16v s = {}, s_lo = {};
 #pragma unroll
     for (int t = 0; t < KSTEPS; ++t) {
       const half8 ka = *reinterpret_cast<const half8*>(Ks + ql * kRow + (((2 * t + half) ^ kswz<HD>(ql)) << 4));
       s = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[t], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qlo[t], s, 0, 0, 0);
+      s_lo = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qlo[t], s_lo, 0, 0, 0);
     }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] += s_lo[e];
     if (kb + 31 > wave_full) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -917,23 +917,26 @@ __global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
     for (int u = 0; u < 2; ++u) {
       uint32_t ph[4], pl[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) split2(s[8 * u + 2 * i], s[8 * u + 2 * i + 1], ph[i], pl[i]);
+      for (int i = 0; i < 4; ++i) split_f16_pair(s[8 * u + 2 * i], s[8 * u + 2 * i + 1], neg1, ph[i], pl[i]);
       const half8 p_hi = __builtin_bit_cast(half8, make_uint4(ph[0], ph[1], ph[2], ph[3]));
       const half8 p_lo = __builtin_bit_cast(half8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
+      half8 va[OT];
 #pragma unroll
       for (int tt = 0; tt < OT; ++tt) {
         const short4v v0 = read_tr4(Vs + vcol[tt] + (16 * u) * kRow);
         const short4v v1 = read_tr4(Vs + vcol[tt] + (16 * u + 8) * kRow);
-        const half8 va = __builtin_bit_cast(half8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-        o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, p_hi, o[tt], 0, 0, 0);
-        o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, p_lo, o[tt], 0, 0, 0);
+        va[tt] = __builtin_bit_cast(half8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
       }
+#pragma unroll
+      for (int tt = 0; tt < OT; ++tt) o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[tt], p_hi, o[tt], 0, 0, 0);
+#pragma unroll
+      for (int tt = 0; tt < OT; ++tt) o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[tt], p_lo, o[tt], 0, 0, 0);
     }
   };
 
-  // Block b's loads of this wave are complete when at most NST - 2 later blocks' are in flight; the barrier
-  // publishes the block and frees the stage of block b - 1, whose reads every wave has waited for. Blocks past
-  // the last are issued too (out of range: no traffic), so the count is a constant.
+  // Stage b's loads of this wave are complete when at most NST - 2 later stages' are in flight; the barrier
+  // publishes it and frees the buffer of stage b - 1, whose reads every wave has waited for. Stages past the
+  // last are issued too (out of range: no traffic), so the count is a constant.
 #pragma unroll
   for (int b = 0; b < NST - 1; ++b) issue(b);
   for (int b = 0; b < nb; ++b) {
@@ -945,22 +948,43 @@ __global__ __launch_bounds__(64 * kUnitWaves, 2) void attn_prefill_mfma_kernel(
     issue(b + NST - 1);
     compute(b);
   }
-  __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): nothing lands in LDS after the waves exit
-
-  if (row_ok && k0 < wave_end) {
-    l = swap_combine32<false>(l);
-    const size_t idx = (static_cast<size_t>(c) * n_q + h) * n_splits + split;
-    if (half == 0) {
-      ws_ml[2 * idx] = m;
-      ws_ml[2 * idx + 1] = l;
-    }
-#pragma unroll
-    for (int tt = 0; tt < OT; ++tt)
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-        reinterpret_cast<float4*>(ws_o + idx * HD + 32 * tt + 8 * a + 4 * half)[0] =
-            make_float4(o[tt][4 * a], o[tt][4 * a + 1], o[tt][4 * a + 2], o[tt][4 * a + 3]);
+  __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): no load lands in the ring from here on
+  if (!row_ok || k0 >= wave_end) return;
+  l = swap_combine32<false>(l);
+  const bool direct = out || xh;  // one split: the result itself; else this split's partial
+  const size_t row = static_cast<size_t>(c) * n_q + h, idx = row * n_splits + split;
+  if (!direct && half == 0) {
+    ws_ml[2 * idx] = m;
+    ws_ml[2 * idx + 1] = l;
   }
+#pragma unroll
+  for (int tt = 0; tt < OT; ++tt)
+#pragma unroll
+    for (int a = 0; a < 4; a += 2) {
+      // dims 8 a + 4 half + i and 8 (a + 1) + 4 half + i of the tile -> lane half h gets all of 8 (a + h) ..
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = o[tt][4 * a + i], y = o[tt][4 * a + 4 + i];
+        const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y),
+                                                        false, false);
+        const unsigned lo = t[0], hi = t[1];  // (a bit cast of a vector element reads element 0 with this compiler)
+        v[i] = __builtin_bit_cast(float, lo);
+        v[4 + i] = __builtin_bit_cast(float, hi);
+      }
+      const int d = 32 * tt + 8 * (a + half);
+      if (direct) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] /= l;
+      }
+      if (xh) {
+        store_x_planes8(xh, xl, static_cast<int64_t>(row * HD + d) / 8, v);
+      } else {
+        float4* dst = reinterpret_cast<float4*>((direct ? out + row * HD : ws_o + idx * HD) + d);
+        dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+        dst[1] = make_float4(v[4], v[5], v[6], v[7]);
+      }
+    }
 }
 
 size_t lds_bytes(int HD, int S) {
@@ -1031,13 +1055,13 @@ int attn_bucket_impl(const float* q, int q_row_stride, const uint16_t* k_cache, 
     return launch_decode(p, hd, n_q / n_kv, q, k_cache, v_cache, ws_ml, ws_o, out, n_kv, L, start, scale, st);
   int rc = Q4_OK;
   if (p.mfma) {
-    const dim3 grid(p.n_splits, n_kv, (p.n_cblk * (n_q / n_kv) + kUnitWaves - 1) / kUnitWaves), block(64 * kUnitWaves);
-    if (hd == 128)
-      hipLaunchKernelGGL(attn_prefill_mfma_kernel<128>, grid, block, 0, st, q, q_row_stride, k_cache, v_cache, ws_ml,
-                         ws_o, C, n_q, n_kv, L, p.S, start, scale);
-    else
-      hipLaunchKernelGGL(attn_prefill_mfma_kernel<64>, grid, block, 0, st, q, q_row_stride, k_cache, v_cache, ws_ml,
-                         ws_o, C, n_q, n_kv, L, p.S, start, scale);
+    // one split: the kernel writes the result itself, in 16-byte stores
+    const bool direct = p.n_splits == 1 && (xh ? aligned(xh, 16) && aligned(xl, 16) : aligned(out, 16));
+    const dim3 grid(p.n_splits, n_kv, (p.n_cblk * (n_q / n_kv) + kUnits - 1) / kUnits), block(64 * kUnits);
+    const auto fn = hd == 128 ? attn_prefill_mfma_kernel<128> : attn_prefill_mfma_kernel<64>;
+    hipLaunchKernelGGL(fn, grid, block, 0, st, q, q_row_stride, k_cache, v_cache, ws_ml, ws_o, C, n_q, n_kv, L, p.S,
+                       start, scale, direct ? out : nullptr, direct ? xh : nullptr, xl);
+    if (direct) return launch_status();
     rc = launch_status();
   } else if (hd == 128) {
     if (p.S == 32) rc = launch_split<128, 32>(p, q, q_row_stride, k_cache, v_cache, ws_ml, ws_o, C, n_q, n_kv, L, start, scale, st);
