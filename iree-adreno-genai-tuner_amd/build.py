@@ -1,4 +1,4 @@
-"""Build the gfx950 library libq4llm.so (and the native runner) in-tree with hipcc.
+"""Build the gfx950 library libq4llm.so, the native runner and the torch call module in-tree.
 
     python iree-adreno-genai-tuner_amd/build.py [--jobs N]
 
@@ -9,10 +9,12 @@ tree to the machine that runs it; nothing is installed.
 
 import argparse
 import concurrent.futures as cf
+import importlib.util
 import os
 import pathlib
 import subprocess
 import sys
+import sysconfig
 
 PKG = pathlib.Path(__file__).resolve().parent
 ROOT = PKG.parent
@@ -46,6 +48,24 @@ def _compile(src: pathlib.Path, obj: pathlib.Path) -> None:
         print(err, file=sys.stderr)
 
 
+def build_torch_module() -> pathlib.Path:
+    """lib/_q4torch.so (csrc/q4_torch.cpp): host code over libq4llm.so and the installed torch's headers."""
+    torch_dir = pathlib.Path(importlib.util.find_spec("torch").submodule_search_locations[0])
+    out = LIB / "_q4torch.so"
+    tmp = LIB / "_q4torch.so.tmp"
+    inc = torch_dir / "include"
+    cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__",
+           "-DUSE_ROCM", "-isystem", str(inc), "-isystem", str(inc / "torch/csrc/api/include"), "-isystem",
+           "/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{ROOT / 'include'}",
+           str(CSRC / "q4_torch.cpp"), "-o", str(tmp), f"-L{LIB}", "-lq4llm", f"-L{torch_dir / 'lib'}", "-ltorch_python",
+           "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"torch module build failed:\n{r.stderr}")
+    os.replace(tmp, out)
+    return out
+
+
 def build(jobs: int = 8, verbose: bool = True) -> pathlib.Path:
     """Compile every source and link lib/libq4llm.so; returns the library path."""
     LIB.mkdir(exist_ok=True)
@@ -70,6 +90,7 @@ def build(jobs: int = 8, verbose: bool = True) -> pathlib.Path:
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"runner build failed:\n{r.stderr}")
+    build_torch_module()
     if verbose:
         print(f"built {out} ({len(srcs)} sources)")
     return out

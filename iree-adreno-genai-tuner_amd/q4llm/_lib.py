@@ -125,6 +125,21 @@ class _Lib:
 LIB = _Lib()
 
 
+def native_calls():
+    """The _q4torch module (csrc/q4_torch.cpp: the ordinary tensor calls in native code, each returning
+    None for what it leaves to the Python wrappers), or None where it is not built for this torch."""
+    import importlib.machinery
+    import importlib.util
+    path = PKG / "lib" / "_q4torch.so"
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_q4torch", str(path))
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_q4torch", loader))
+        loader.exec_module(mod)
+        return mod
+    except ImportError:
+        return None
+
+
 def exported_symbols():
     """Names declared in include/q4llm.h (parsed from the header text)."""
     import re

@@ -86,6 +86,11 @@ class QLinear(nn.Module):
 
     def forward(self, x, residual=None, out=None):
         """x [M, K] fp32 -> [M, N] fp32 (+ residual); M == 1 is the decode GEMV."""
+        if out is None:
+            p = self._parameters
+            y = ops.linear_call(p.get("qweight"), p.get("scales"), x, self.group, residual, True)
+            if y is not None:
+                return y
         x = x.reshape(-1, self.k).float().contiguous()
         if x.shape[0] == 1:
             y = ops.q4_gemv(self.qweight, self.scales, x[0], self.group, residual=None if residual is None

@@ -125,3 +125,52 @@ def test_attn_prefill_units_and_splits(dev, kernel_override, C, start, L, nq, nk
     # scores of fp16 hi + lo queries: 2^-22 sum |q k| each, the same again for the fp32 sums; P likewise
     smax = (q.abs().double().sum(-1).max() * 4.0 * abs(scale)).item()
     assert (out.cpu().double() - ref).abs().max().item() <= 5.0 * (2.0 ** -20 * max(smax, 1.0)) + 1e-6
+
+
+def test_native_calls_match_python_wrappers(dev, monkeypatch):
+    """The native calls and the Python wrappers they stand in for give the same bits and the same errors,
+    on the current stream; operands the native code leaves alone (views that need a copy, an `out`, other
+    shapes) still work."""
+    from q4llm import llama_q4 as Q
+    g = torch.Generator(device=dev).manual_seed(3)
+
+    def rnd(*s):
+        return torch.randn(*s, device=dev, generator=g)
+
+    lin = Q.QLinear(rnd(96, 256) * 0.02, 32)
+    qw, sc = lin.qweight, lin.scales
+    x1, x5, x40, res = rnd(1, 256), rnd(5, 256), rnd(40, 256), rnd(40, 96)
+    kc, vc, q = rnd(64, 2, 64).half(), rnd(64, 2, 64).half(), rnd(3, 4, 64)
+    st = torch.tensor([5], dtype=torch.int32, device=dev)
+    a, b = rnd(33, 64).half(), rnd(24, 128).half()[:, :64]
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device=dev)
+
+    def results():
+        side = torch.cuda.Stream(dev)
+        side.wait_stream(torch.cuda.current_stream(dev))
+        out16 = torch.empty(96, dtype=torch.float16, device=dev)
+        with torch.cuda.stream(side):
+            r = [ops.q4_gemv(qw, sc, x1, 32), ops.q4_gemv(qw, sc, x1[0].half(), 32, out_dtype=torch.float16),
+                 ops.q4_gemv(qw, sc, x1[0], 32, residual=res[0]), ops.q4_gemv(qw, sc, x1[0].half(), 32, out=out16),
+                 ops.q4_gemv(qw, sc, rnd(256, 2)[:, 0] * 0 + x1[0], 32), lin(x1), lin(x1[0]), lin(x5, residual=res[:5]),
+                 lin(x40, residual=res), lin(x40.half()), lin(x40[None]), lin(rnd(256, 40).t() * 0 + x40),
+                 ops.q4_linear(x1, qw, sc, 32), ops.attn_bucket(q, kc, vc, 64, st, 0.1),
+                 ops.attn_bucket(q[:1], kc, vc, 33, st, 0.1, workspace=ws),
+                 ops.attn_bucket(q.transpose(0, 1).contiguous().transpose(0, 1), kc, vc, 64, st, 1),
+                 ops.gemm_f16_nt(a, b), ops.gemm_f16_nt_ws(a, b, workspace=ws), ops.gemm_f16_nt(a[:1], b)]
+        assert r[3] is out16
+        torch.cuda.current_stream(dev).wait_stream(side)
+        return r
+
+    native = results()
+    for name in ("_gemv", "linear_call", "_attn", "_gemm"):
+        monkeypatch.setattr(ops, name, ops._left_to_python)
+    for i, (u, v) in enumerate(zip(native, results())):
+        assert u.shape == v.shape and u.dtype == v.dtype and torch.equal(u, v), i
+    monkeypatch.undo()
+    for bad in (lambda: ops.q4_gemv(qw, sc, x1.double(), 32), lambda: ops.q4_gemv(qw, sc, x1[:, :64], 32),
+                lambda: ops.q4_gemv(qw, sc.float(), x1, 32), lambda: ops.q4_linear(x5[:, :128], qw, sc, 32),
+                lambda: ops.gemm_f16_nt(a, b.float()), lambda: ops.gemm_f16_nt(a.t(), b),
+                lambda: lin(x5, residual=res), lambda: ops.q4_gemv(qw, sc, x1, 48)):
+        with pytest.raises(ValueError):
+            bad()
