@@ -28,6 +28,7 @@
 #include "q4_internal.h"
 
 #include <algorithm>
+#include <cstdint>
 #include <cstdlib>
 #include <type_traits>
 
@@ -455,13 +456,15 @@ struct TileCfg {
 constexpr TileCfg kTiles[] = {
     {256, 256, 2, 4, 2, 64},        // 0: 8 waves of 128x64, 2 stages of K 64 (128 KB LDS)
     {128, 128, 2, 2, 2, 64},        // 1: 4 waves of 64x64, 2 stages (64 KB, two workgroups per CU)
-    {128, 128, 2, 2, 4, 64, true},  // 2: 4 waves of 64x64, 4 stages (128 KB), pipelined substeps
-    {64, 96, 2, 3, 4, 64, true},    // 3: 6 waves of 32x32, 4 stages (81 KB), pipelined: M = 256, N = 5120 on 216 CUs
-    {128, 64, 2, 2, 4, 64},         // 4: 4 waves of 64x32, 4 stages (96 KB)
-    {64, 64, 2, 2, 4, 64},          // 5: 4 waves of 32x32, 4 stages (64 KB)
-    {128, 160, 2, 5, 4, 64, true},  // 6: 10 waves of 64x32, 4 stages (145 KB), pipelined: M = 1024, N = 5120
-                                    //    in exactly 256 tiles
+    {128, 128, 2, 2, 4, 64, true},  // 2: 4 waves of 64x64, 4 stages (128 KB), pipelined (entry 5 with one wave per
+                                    //    SIMD: for sweeps, the rule never takes it)
+    {64, 64, 2, 2, 4, 64},          // 3: 4 waves of 32x32, 4 stages (64 KB, two workgroups per CU)
+    {128, 160, 2, 5, 4, 64, true},  // 4: 10 waves of 64x32, 4 stages (145 KB), pipelined
+    {128, 128, 4, 2, 4, 64, true},  // 5: 8 waves of 32x64, 4 stages (128 KB), pipelined
+    {256, 128, 4, 2, 3, 64, true},  // 6: 8 waves of 64x64, 3 stages (144 KB), pipelined
+    {64, 128, 2, 4, 4, 64, true},   // 7: 8 waves of 32x32, 4 stages (96 KB), pipelined
 };
+constexpr int kSmallEntry = 3, kWideEntry = 2;  // the 64x64 tile; the 128x128 one that K splits are sized by below
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
 using GemmFn = void (*)(const uint16_t*, const uint16_t*, uint16_t*, int, int, int, int, int, int, int, int, int, int,
@@ -478,60 +481,28 @@ constexpr size_t gemm_lds() {
   return GemmCfg<t.bm, t.bn, t.wgm, t.wgn, t.nst, t.bk>::kLds;
 }
 constexpr GemmFn kGemmFns[] = {gemm_fn<0>(), gemm_fn<1>(), gemm_fn<2>(), gemm_fn<3>(),
-                               gemm_fn<4>(), gemm_fn<5>(), gemm_fn<6>()};
+                               gemm_fn<4>(), gemm_fn<5>(), gemm_fn<6>(), gemm_fn<7>()};
 constexpr size_t kGemmLds[] = {gemm_lds<0>(), gemm_lds<1>(), gemm_lds<2>(), gemm_lds<3>(),
-                               gemm_lds<4>(), gemm_lds<5>(), gemm_lds<6>()};
+                               gemm_lds<4>(), gemm_lds<5>(), gemm_lds<6>(), gemm_lds<7>()};
 static_assert(sizeof(kGemmFns) / sizeof(kGemmFns[0]) == kNumTiles, "one kernel per tile entry");
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Fixed rule, from sweeps of every entry (and K splits of 1-8) over the config-3 shapes on one
-// MI355X (graph replays, weights rotated past the MALL):
-//   * M >= 512: 256x256 when that alone fills the 256 CUs (4096^3: 1.05 PFLOP/s); else the pipelined
-//     128x160 entry when its tiles make one round of 240-256 workgroups (1024x5120x3072: 256 tiles,
-//     46.0 -> 41.7 us against 128x128); else 128x128 with two workgroups per CU (2048x3072x8192:
-//     117 us; 128x160 there gives 320 tiles, 179 us, and 128x192 256 tiles, 129 us); K splits only
-//     lost here;
-//   * M < 512 with a workspace (gemm_f16_nt_ws): the pipelined 128x128 entry with K split so the
-//     tiles times the split come closest to 256 workgroups (256x5120x3072: 80 tiles x 3, 23.1 us;
-//     256x3072x8192: 48 x 5, 29 us; 256x16384x3072: 256 x 1, 40 us);
-//   * M < 512 without one: the largest 4-stage tile that still gives >= 160 workgroups (pipelined
-//     128x128, then 64x96 where it fills the CUs in one round, then 128x64, 64x64).
-// Measured and not in the list: whole-256-row tiles (256x64, 64x256, 256x32), 4 waves of 128x128 on
-// 256x256 tiles (2 stages of K 64, or 4-5 stages of K 32) and of 64x128 / 128x64, 8 waves on 256x128
-// and 128x256, K steps of 128, the plain schedule on the 4-stage 128x128 and 64x96 tiles (the
-// pipelined ones replace them), the pipelined schedule on the 8-wave 256x256 and the two-workgroup
-// 128x128 entries, and a ping-pong schedule of two 4-wave groups on 256x256: each equal or slower on
-// every config-3 shape.
 // Problems under 4 GFLOP (under ~2 us of matrix-core time at the dense peak) are set by latency and
-// by how many CUs stream at once, not by the tile's operand reuse.
+// by how many CUs stream at once, not by the tile's operand reuse: the 64x64 entry, the K split of
+// gemm_split_plan (swept on every entry and splits of 1-32: S1 1024^3 15.3 -> 9.0 us, S3 15.3 -> 8.3,
+// S5 19.5 -> 12.0, S8 12.7 -> 7.2), unless its tiles need more than the 512 workgroups that run at once.
 bool small_problem(int64_t M, int64_t N, int64_t K) { return 2.0 * M * N * K < 4e9; }
-
-int choose_tile(int64_t M, int64_t N, int64_t K, bool split_ok) {
-  const int ov = debug_override(Q4_DBG_GEMM_TILE);
-  if (ov >= 0 && ov < kNumTiles) return ov;
-  (void)split_ok;
-  // small problems (the reference's S1-S6 and S8): 64x64, the K split below (swept on every entry and
-  // splits of 1-32: S1 1024^3 15.3 -> 9.0 us, S3 15.3 -> 8.3, S5 19.5 -> 12.0, S8 12.7 -> 7.2)
-  if (small_problem(M, N, K)) return 5;
-  auto tiles = [&](int i) { return cdiv(M, kTiles[i].bm) * cdiv(N, kTiles[i].bn); };
-  if (M >= 512) return tiles(0) >= 256 ? 0 : (tiles(6) >= 240 && tiles(6) <= 256 ? 6 : 1);
-  if (split_ok && N % 4 == 0) return 2;
-  if (tiles(2) >= 160) return 2;
-  // 64x96 when it covers the CUs in one round (256x5120x3072: 160 workgroups of 128x64 -> 216 of 64x96,
-  // 17% fewer bytes per CU, 27.6 -> 23.6 us)
-  if (tiles(3) >= 160 && tiles(3) <= 256) return 3;
-  for (int i : {4, 5})
-    if (tiles(i) >= 160) return i;
-  return 5;
+bool latency_bound(int64_t M, int64_t N, int64_t K) {
+  return small_problem(M, N, K) && cdiv(M, 64) * cdiv(N, 64) <= 512;
 }
 
 }  // namespace
 
-// K split of tile entry ti: n_split K ranges of nk_split K steps each (the last may be shorter, none
-// empty); {1, 0} for no split. Only when N % 4 == 0 (the reduce kernel's four-column rows): M < 512
-// takes the split that brings the workgroups closest to 256 without exceeding it, each range at least
-// four K steps. The Q4_DBG_GEMM_SPLIT override forces a split count for sweeps.
+// K split of tile entry ti by size alone: n_split K ranges of nk_split K steps each (the last may be
+// shorter, none empty); {1, 0} for no split. Only when N % 4 == 0 (the reduce kernel's four-column rows):
+// M < 512 takes the split that brings the workgroups closest to 256 without exceeding it, each range at
+// least four K steps. The Q4_DBG_GEMM_SPLIT override forces a split count for sweeps.
 struct GemmSplit {
   int n_split, nk_split;
 };
@@ -554,10 +525,91 @@ GemmSplit gemm_split_plan(int64_t M, int64_t N, int64_t K, int ti) {
   return p;
 }
 
-size_t gemm_split_bytes(int64_t M, int64_t N, int64_t K, int ti) {
-  const GemmSplit sp = gemm_split_plan(M, N, K, ti);
-  return sp.n_split > 1 ? static_cast<size_t>(sp.n_split) * M * N * sizeof(float) : 0;
+namespace {
+
+// A tile entry with its K split.
+struct GemmPlan {
+  int tile;
+  GemmSplit split;
+  size_t bytes(int64_t M, int64_t N) const {
+    return split.n_split > 1 ? static_cast<size_t>(split.n_split) * M * N * sizeof(float) : 0;
+  }
+};
+
+// Estimated time (us) of `wgs` workgroups of `steps` K steps on entry ti: rounds of at most `cap` workgroups
+// (those that run at once), each costing its start and, per step, a time that grows with how many of them
+// load. Fitted (least squares of the relative error, median 4%) to 150 shapes of M 17-4096, N 64-5120, K
+// 64-8192 with splits of 1-16, graph replays over rotated operands on one MI355X. Entry 2 is left out.
+double tile_time(int ti, int64_t wgs, int64_t steps) {
+  struct Rate {
+    double fixed, round, step, load;
+    int cap;
+  };
+  constexpr Rate kRates[kNumTiles] = {{8.9, 1.6, 1.346, 0.036, 256}, {5.7, 3.4, 0.575, 0.182, 512}, {0, 0, 0, 0, 0},
+                                      {3.2, 1.5, 0.322, 0.061, 512}, {5.1, 2.1, 0.568, 0.110, 256},
+                                      {4.5, 2.6, 0.443, 0.086, 256}, {6.2, 1.5, 0.740, 0.147, 256},
+                                      {3.5, 2.0, 0.354, 0.041, 256}};
+  const Rate& r = kRates[ti];
+  const int64_t full = wgs / r.cap, rest = wgs % r.cap;
+  double us = r.fixed + static_cast<double>(full - (rest ? 0 : 1)) * r.round;
+  us += static_cast<double>(full * steps) * (r.step + r.load * r.cap / 256.0);
+  if (rest) us += static_cast<double>(steps) * (r.step + r.load * static_cast<double>(rest) / 256.0);
+  return us;
 }
+
+// The rule: latency-bound problems as above; else the cheapest entry by tile_time, with a K split of up to
+// 16 ranges of at least four steps where N % 4 == 0 and its partials fit `part_bytes` (their write, read and
+// launch: 3.3 us + 1.08 us per million; 5% in favour of no split, the estimate's error: 2048x3072x8192 in two
+// ranges was estimated at par and measured 121.8 us against 117.7). Against the fixed size rules before it
+// (us, same run): 256x3072x8192 28.9 -> 25.6, 512x3072x8192 83.9 -> 40.6, 512x5120x3072 39.1 -> 28.3,
+// 1024x3072x3072 38.9 -> 28.8, 3000x3000x3000 107 -> 92, 1536x1536x4096 47.3 -> 35.1, 256x16384x3072 38.1 ->
+// 34.0, 607x5172x64 8.0 -> 6.3; over the 150 shapes it is 1.6% off the best entry and split of each.
+// Measured and not in the list: whole-256-row tiles (256x64, 64x256, 256x32), 64x96 and 128x64, 4 waves of
+// 128x128 on 256x256 tiles (2 stages of K 64, or 4-5 stages of K 32) and of 64x128 / 128x64, 128x256, K
+// steps of 128, the plain schedule on the 4-stage tiles, the pipelined schedule on the 256x256 and the
+// two-workgroup 128x128 entries, and a ping-pong schedule of two 4-wave groups on 256x256.
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, size_t part_bytes) {
+  const int ov = debug_override(Q4_DBG_GEMM_TILE);
+  const bool forced = ov >= 0 && ov < kNumTiles;
+  if (forced || debug_set(Q4_DBG_GEMM_SPLIT) || latency_bound(M, N, K)) {
+    const int ti = forced ? ov : latency_bound(M, N, K) ? kSmallEntry : kWideEntry;
+    const GemmPlan p{ti, gemm_split_plan(M, N, K, ti)};
+    return p.bytes(M, N) <= part_bytes ? p : GemmPlan{ti, {1, 0}};
+  }
+  GemmPlan best{kSmallEntry, {1, 0}};
+  double best_us = 1e30;
+  for (int ti = 0; ti < kNumTiles; ++ti) {
+    if (ti == kWideEntry) continue;
+    const TileCfg& t = kTiles[ti];
+    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn), nk = cdiv(K, t.bk);
+    // a split is of use only while one range fewer leaves workgroup slots idle
+    for (int64_t want = 1; want <= 16 && (want == 1 || tiles * (want - 1) < 256); ++want) {
+      const int64_t nk_s = cdiv(nk, want), S = cdiv(nk, nk_s);
+      const GemmPlan p{ti, {static_cast<int>(S), S > 1 ? static_cast<int>(nk_s) : 0}};
+      if (S != want || (S > 1 && (N % 4 || M <= 1 || nk_s < 4 || p.bytes(M, N) > part_bytes))) continue;
+      double us = tile_time(ti, tiles * S, nk_s);
+      if (S > 1) us = 1.05 * (us + 3.3 + 1.08e-6 * static_cast<double>(S * M * N));
+      if (us < best_us) best_us = us, best = p;
+    }
+  }
+  return best;
+}
+
+// Whether gemm_f16_nt_ws takes this workspace: all that the split by size alone needs (latency-bound
+// problems and M < 512; none from there on), or all that the plan asks for. With less than the plan asks
+// for, the call runs the best plan that fits.
+bool gemm_workspace_ok(int64_t M, int64_t N, int64_t K, const void* ws, size_t ws_bytes) {
+  if (M == 1) return true;
+  const bool usable = ws && aligned(ws, 16);
+  auto holds = [&](size_t need) { return need == 0 || (usable && ws_bytes >= need); };
+  if (!debug_set(Q4_DBG_GEMM_TILE) && !debug_set(Q4_DBG_GEMM_SPLIT)) {
+    const int ti = small_problem(M, N, K) ? kSmallEntry : kWideEntry;
+    if (holds(GemmPlan{ti, gemm_split_plan(M, N, K, ti)}.bytes(M, N))) return true;
+  }
+  return holds(gemm_plan(M, N, K, SIZE_MAX).bytes(M, N));
+}
+
+}  // namespace
 
 int gemm_f16_launch(const uint16_t* A, const uint16_t* B, uint16_t* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                     int64_t ldb, int64_t ldc, int cfg, hipStream_t st, float* part = nullptr, size_t part_bytes = 0) {
@@ -585,7 +637,10 @@ int gemm_f16_launch(const uint16_t* A, const uint16_t* B, uint16_t* C, int64_t M
     else go(std::integral_constant<int, 8>{});
     return launch_status();
   }
-  const int ti = cfg >= 0 && cfg < kNumTiles ? cfg : choose_tile(M, N, K, part != nullptr);
+  // a buffer that the partials cannot use counts as none
+  const size_t room = part && aligned(part, 16) ? part_bytes : 0;
+  const GemmPlan plan = cfg >= 0 && cfg < kNumTiles ? GemmPlan{cfg, {1, 0}} : gemm_plan(M, N, K, room);
+  const int ti = plan.tile;
   const TileCfg& t = kTiles[ti];
   const int tiles_m = static_cast<int>(cdiv(M, t.bm)), tiles_n = static_cast<int>(cdiv(N, t.bn));
   const int ntiles = tiles_m * tiles_n;
@@ -594,12 +649,7 @@ int gemm_f16_launch(const uint16_t* A, const uint16_t* B, uint16_t* C, int64_t M
     Q4_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kGemmFns[ti]),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
   }
-  GemmSplit sp{1, 0};
-  if (part) {
-    sp = gemm_split_plan(M, N, K, ti);
-    if (sp.n_split > 1 && (part_bytes < static_cast<size_t>(sp.n_split) * M * N * sizeof(float) || !aligned(part, 16)))
-      return Q4_ERR_WORKSPACE;
-  }
+  const GemmSplit sp = plan.split;
   const int grid = ntiles * sp.n_split;
   const int remap = (grid % 8 == 0) ? 1 : 0;
   hipLaunchKernelGGL(kGemmFns[ti], dim3(grid, 1), dim3(64 * t.wgm * t.wgn), lds, st, A, B, C, (int)M, (int)N, (int)K,
@@ -621,7 +671,7 @@ int gemm_f16_launch(const uint16_t* A, const uint16_t* B, uint16_t* C, int64_t M
 // Workspace bytes gemm_f16_nt_ws uses for this shape (0: no K split).
 size_t gemm_f16_ws_bytes(int64_t M, int64_t N, int64_t K) {
   if (M == 1) return 0;
-  return gemm_split_bytes(M, N, K, choose_tile(M, N, K, true));
+  return gemm_plan(M, N, K, SIZE_MAX).bytes(M, N);
 }
 
 int gemm_f16_num_tiles() { return kNumTiles; }
@@ -665,7 +715,7 @@ extern "C" int gemm_f16_nt_ws(const uint16_t* A, const uint16_t* B, uint16_t* C,
                               int64_t lda, int64_t ldb, int64_t ldc, void* workspace, size_t workspace_bytes,
                               void* stream) {
   if (int st = gemm_args(A, B, C, M, N, K, lda, ldb, ldc)) return st;
-  if (M > 1 && !workspace && q4::gemm_f16_ws_bytes(M, N, K) > 0) return Q4_ERR_WORKSPACE;
+  if (!q4::gemm_workspace_ok(M, N, K, workspace, workspace_bytes)) return Q4_ERR_WORKSPACE;
   return q4::gemm_f16_launch(A, B, C, M, N, K, lda, ldb, ldc, -1, q4::as_stream(stream),
                              static_cast<float*>(workspace), workspace_bytes);
 }

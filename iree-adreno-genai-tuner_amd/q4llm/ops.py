@@ -276,7 +276,12 @@ def gemm_f16_nt_ws(a, b, out=None, workspace=None):
     if out is None:
         out = torch.empty(m, n, dtype=torch.float16, device=a.device)
     if workspace is None:
-        workspace = torch.empty(max(gemm_f16_nt_ws_bytes(m, n, k), 16), dtype=torch.uint8, device=a.device)
+        try:
+            workspace = torch.empty(max(gemm_f16_nt_ws_bytes(m, n, k), 16), dtype=torch.uint8, device=a.device)
+        except torch.OutOfMemoryError:
+            if m < 512:
+                raise
+            workspace = torch.empty(16, dtype=torch.uint8, device=a.device)  # from 512 rows on, any size is taken
     _need(workspace, "workspace", torch.uint8, None)
     LIB.call("gemm_f16_nt_ws", ptr(a), ptr(b), ptr(out), m, n, k, a.stride(0), b.stride(0), out.stride(0),
              ptr(workspace), workspace.numel(), stream_of(a.device))

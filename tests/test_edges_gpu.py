@@ -6,6 +6,7 @@ import torch
 
 from oracle import llama_q4_ref as R
 from q4llm import ops
+from q4llm._lib import LIB
 
 pytestmark = pytest.mark.gpu
 
@@ -125,6 +126,36 @@ def test_attn_prefill_units_and_splits(dev, kernel_override, C, start, L, nq, nk
     # scores of fp16 hi + lo queries: 2^-22 sum |q k| each, the same again for the fp32 sums; P likewise
     smax = (q.abs().double().sum(-1).max() * 4.0 * abs(scale)).item()
     assert (out.cpu().double() - ref).abs().max().item() <= 5.0 * (2.0 ** -20 * max(smax, 1.0)) + 1e-6
+
+
+@pytest.mark.parametrize("M,N,K", [(511, 3076, 2056), (512, 3076, 2056), (257, 2052, 8192), (700, 2243, 3000),
+                                   (2049, 1030, 1032), (33, 8196, 8200), (1023, 513, 4104), (2600, 3000, 264),
+                                   (2, 4096, 65536), (1536, 1540, 4096), (4096, 2052, 64)])
+def test_gemm_plan_and_workspace_sizes(dev, M, N, K):
+    """Sizes on both sides of the GEMM rule's lines (latency-bound, the tiles chosen by estimated time, the K
+    split), each with the workspace it asks for, with one that only a smaller plan fits, and with none where
+    the split by size alone needs none."""
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    a = torch.randn(M, K, device=dev, generator=g).half()
+    b = torch.randn(N, K, device=dev, generator=g).half()
+    ref = a.double() @ b.double().t()
+    # fp32 sums of K products (their errors add like a random walk; 8 sigma) and the fp16 result
+    bound = 2.0 ** -11 * ref.abs() + 8 * K ** 0.5 * 2.0 ** -24 * (K ** 0.5) + 2.0 ** -14
+    f = LIB.raw("gemm_f16_nt_ws")
+    st = torch.cuda.current_stream(dev).cuda_stream
+
+    def check(c, what):
+        assert ((c.double() - ref).abs() <= bound).all(), what
+
+    check(ops.gemm_f16_nt(a, b), "no workspace entry")
+    need = ops.gemm_f16_nt_ws_bytes(M, N, K)
+    for nbytes in {need, max(need, 16) + 48, need // 2, 0} if M >= 512 else {need, need + 48}:
+        ws = torch.full((nbytes + 64,), 255, dtype=torch.uint8, device=dev)
+        c = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+        assert f(ops.ptr(a), ops.ptr(b), ops.ptr(c), M, N, K, K, K, N, ops.ptr(ws) if nbytes else None, nbytes, st) == 0
+        check(c, nbytes)
+        assert (ws[nbytes:] == 255).all()
+    check(ops.gemm_f16_nt_ws(a, b), "its own workspace")
 
 
 def test_native_calls_match_python_wrappers(dev, monkeypatch):
