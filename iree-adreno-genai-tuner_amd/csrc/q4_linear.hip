@@ -861,19 +861,29 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void q4_linear_ws_kernel(
         }
         if (row < M && col < N) {
           const int64_t o = static_cast<int64_t>(row) * N + col;
-          if (n_split > 1) P[static_cast<int64_t>(ksp) * M * N + o] = acc[i][j][e];
+          if (n_split > 1) P[ksp * ((static_cast<int64_t>(M) * N + 3) & ~int64_t{3}) + o] = acc[i][j][e];
           else Y[o] = R ? R[o] + acc[i][j][e] : acc[i][j][e];
         }
       }
 }
 
-// y = residual + sum_s P[s] over n = M N / 4 float4 elements, the splits added in ascending order
-// (fixed, so results do not depend on scheduling); y may alias the residual.
+// y = residual + sum_s P[s] over `total` floats, four to a thread, the splits added in ascending order
+// (fixed, so results do not depend on scheduling); y may alias the residual. Each P[s] starts on a whole
+// float4 (total rounded up); a last element of fewer than four floats is read whole and written one by one.
 __global__ __launch_bounds__(256) void linear_reduce_kernel(const float4* __restrict__ P, const float4* R, float4* Y,
-                                                            int64_t n, int n_split) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+                                                            int64_t total, int n_split) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, n = (total + 3) / 4;
   if (i >= n) return;
   float4 a = sum_partials4(P + i, n, n_split);
+  if (4 * i + 4 > total) {
+    const float v[3] = {a.x, a.y, a.z};
+    const float* r = reinterpret_cast<const float*>(R);
+    float* y = reinterpret_cast<float*>(Y);
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      if (4 * i + j < total) y[4 * i + j] = r ? r[4 * i + j] + v[j] : v[j];
+    return;
+  }
   if (R) {
     const float4 r = R[i];
     a = make_float4(r.x + a.x, r.y + a.y, r.z + a.z, r.w + a.w);
@@ -1007,9 +1017,12 @@ LinearSplit linear_split_plan(int64_t M, int64_t N, int64_t K, int group) {
   return p;
 }
 
+// one K range's partials: [M, N] fp32, rounded up to whole float4s
+static size_t plane_bytes(int64_t M, int64_t N) { return static_cast<size_t>((M * N + 3) / 4) * 16; }
+
 size_t linear_split_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
   const LinearSplit p = linear_split_plan(M, N, K, group);
-  return p.n_split > 1 ? static_cast<size_t>(p.n_split) * M * N * sizeof(float) : 0;
+  return p.n_split > 1 ? p.n_split * plane_bytes(M, N) : 0;
 }
 
 namespace {
@@ -1018,71 +1031,71 @@ struct LinPlan {
   int tile;
   LinearSplit split;
   size_t part_bytes(int64_t M, int64_t N) const {
-    return split.n_split > 1 ? static_cast<size_t>(split.n_split) * M * N * sizeof(float) : 0;
+    return split.n_split > 1 ? split.n_split * plane_bytes(M, N) : 0;
   }
 };
 
 // Estimated time (us) of `wgs` workgroups of `steps` 64-k stages each on tile entry `ti`: rounds of at most
-// kRound workgroups, whose stage time grows with how many of them run (the matrix cores' clock and the
-// L2 are shared). Constants fitted to one MI355X, graph replays over rotated weights, group 128 | 32:
-//   64x256 (8 waves of 32x64):   48 workgroups 0.86 | 1.29 us a stage, 160 1.03 | 1.41, 256 1.16 | 1.60
-//   128x256 (8 waves of 64x64):  40 workgroups 1.37 | 2.13, 128 1.58 | 2.29, 256 1.92 | 2.63
-//   32x64 (three per CU):        480 workgroups 0.56 | 0.63, 768 0.83 | 0.92
+// `cap` workgroups, each stage's time growing with how many of them run (the matrix cores' clock and the
+// L2 are shared). Fitted (relative error 3% in the median, 10% at the 90th percentile) to 400 shapes of M
+// 33-1024, N 256-16384, K 128-8192 at groups 128 and 32, splits of 1-16, graph replays over rotated weights.
 double tile_time(int ti, int64_t wgs, int64_t steps, int group) {
   struct Rate {
-    double fixed, a, b;
-    int round;
+    double fixed, round, step, load;
+    int cap;
   };
-  constexpr Rate kRates[2][3] = {{{6.0, 0.30, 0.00070, 768}, {7.0, 0.82, 0.00133, 256}, {8.0, 1.28, 0.0025, 256}},
-                                 {{6.0, 0.36, 0.00073, 768}, {7.0, 1.23, 0.00145, 256}, {8.0, 2.03, 0.0023, 256}}};
+  constexpr Rate kRates[2][3] = {{{5.7, 1.0, 0.352, 0.112, 768}, {7.2, 0, 0.801, 0.201, 256}, {8.7, 0, 1.318, 0.200, 256}},
+                                 {{5.7, 1.0, 0.397, 0.125, 768}, {7.3, 0, 1.258, 0.167, 256}, {8.7, 0, 2.030, 0.100, 256}}};
   const Rate& r = kRates[group >= 128 ? 0 : 1][ti];
-  double t = r.fixed;
-  for (; wgs > 0; wgs -= r.round) t += steps * (r.a + r.b * static_cast<double>(std::min<int64_t>(wgs, r.round)));
-  return t;
+  const int64_t full = wgs / r.cap, rest = wgs % r.cap;
+  double us = r.fixed + static_cast<double>(full - (rest ? 0 : 1)) * r.round;
+  us += static_cast<double>(full * steps) * (r.step + r.load * r.cap / 256.0);
+  if (rest) us += static_cast<double>(steps) * (r.step + r.load * static_cast<double>(rest) / 256.0);
+  return us;
 }
 
-// The cheapest tile by tile_time, with a K split (pipelined tiles; whole groups, at least four stages, at
-// most eight splits) where the planes may be followed by up to `part_bytes` of partials: their write and
-// read cost 8 S M N bytes at 4.5 TB/s and the reduce launch 2.5 us. Against the 64x64 and 32x64 tiles that
-// ran all of these before (us, with the x split): 512x5120x3072 78.8 -> 52.4, 512x16384x3072 197 -> 100
-// (group 32: 241 -> 135), 1024x5120x3072 127 -> 83, 1024x16384x3072 375 -> 190.
-LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes) {
+// The cheapest tile by tile_time, with a K split of up to 16 (pipelined tiles; whole groups, at least two
+// stages) whose partials fit `part_bytes`: their write and read cost 1.45 us per million, the launch that adds
+// them 2.0 us (none where the next kernel does it), and the estimate's error 5% in favour of no split.
+// Against the 64x64 and 32x64 tiles that ran all of these before (us, with the x split): 512x5120x3072
+// 78.8 -> 52.4, 512x16384x3072 197 -> 100 (group 32: 241 -> 135), 1024x5120x3072 127 -> 83, 1024x16384x3072
+// 375 -> 190. Against a split of every M <= 256 into about 256 workgroups of 64x256 (linear_split_plan), short
+// K: 250x3560x384 17.6 -> 10.3, 250x3072x1024 21.0 -> 16.0, 100x8192x1024 21.5 -> 15.5, 33x16384x640 16.5 -> 11.6.
+LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool reduce) {
   const int64_t nk = K / 64, gst = group > 64 ? group / 64 : 1;
   LinPlan best{kSmallTile, {1, 0}};
-  double best_t = 0.0;
+  double best_us = 1e30;
   for (int ti = 0; ti < kNumLinWs; ++ti) {
     const LinWsTile& t = kLinWsTiles[ti];
     const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-    for (int64_t want = 1; want <= (t.pipe ? 8 : 1); ++want) {
+    for (int64_t want = 1; want <= (t.pipe ? 16 : 1) && (want == 1 || tiles * (want - 1) < 256); ++want) {
       int64_t nk_s = (nk + want - 1) / want;
       nk_s = (nk_s + gst - 1) / gst * gst;
       const int64_t S = (nk + nk_s - 1) / nk_s;
-      if (S != want || (S > 1 && (nk_s < 4 || static_cast<size_t>(S) * M * N * sizeof(float) > part_bytes))) continue;
+      const LinPlan p{ti, {static_cast<int>(S), S > 1 ? static_cast<int>(nk_s) : 0}};
+      if (S != want || (S > 1 && (nk_s < 2 || p.part_bytes(M, N) > part_bytes))) continue;
       double us = tile_time(ti, tiles * S, nk_s, group);
-      if (S > 1) us += 2.5 + 8e-6 / 4.5 * static_cast<double>(S * M * N);
-      if ((ti == 0 && S == 1) || us < best_t) {
-        best_t = us;
-        best = LinPlan{ti, {static_cast<int>(S), S > 1 ? static_cast<int>(nk_s) : 0}};
-      }
+      if (S > 1) us = 1.05 * (us + (reduce ? 2.0 : 0.0) + 1.45e-6 * static_cast<double>(S * M * N));
+      if (us < best_us) best_us = us, best = p;
     }
   }
   return best;
 }
 
-// The rule: chunks of at most 256 rows with room for their partials take linear_split_plan where it
-// splits; everything else the cheapest tile.
-LinPlan linear_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes) {
+// The rule: chunks of at most 256 rows whose partials the next kernel adds (a model step) take
+// linear_split_plan where it splits; everything else the cheapest tile.
+LinPlan linear_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool deferred) {
   const LinearSplit sp = linear_split_plan(M, N, K, group);
-  if (sp.n_split > 1 && part_bytes >= linear_split_part_bytes(M, N, K, group)) return LinPlan{kSplitTile, sp};
-  return tile_plan(M, N, K, group, M > 256 ? part_bytes : 0);
+  if (deferred && sp.n_split > 1 && part_bytes >= linear_split_part_bytes(M, N, K, group)) return LinPlan{kSplitTile, sp};
+  return tile_plan(M, N, K, group, deferred && M <= 256 ? 0 : part_bytes, !deferred);
 }
 }  // namespace
 
 // Bytes of partials with which q4_linear_planes takes its fastest plan, outside the model step too
 // (there linear_split_part_bytes: no split past 256 rows).
 size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
-  if (M <= 256) return linear_split_part_bytes(M, N, K, group);
-  return tile_plan(M, N, K, group, SIZE_MAX).part_bytes(M, N);
+  return std::max(linear_split_part_bytes(M, N, K, group),
+                  tile_plan(M, N, K, group, SIZE_MAX, true).part_bytes(M, N));
 }
 
 // The pipelined GEMM on x given as fp16 (hi, lo) planes (store_x_planes layout, [M, K] each);
@@ -1094,9 +1107,11 @@ int q4_linear_planes(const uint16_t* xh, const uint16_t* xl, int64_t M, const in
   if (int e = planes_args(xh, xl, M, qw, sc, N, K, group)) return e;
   if (!y) return Q4_ERR_NULL;
   if (deferred) *deferred = 0;
-  // what the partials and linear_reduce_kernel need: whole float4s, 16-byte alignment, 32-bit indexes
-  const bool can_split = part && (M * N) % 4 == 0 && aligned(part, 16) && aligned(y, 16) && (!res || aligned(res, 16));
-  LinPlan plan = linear_plan(M, N, K, group, can_split ? std::min<size_t>(part_bytes, size_t{1} << 33) : 0);
+  // what the partials and linear_reduce_kernel (a caller's next kernel: whole float4s too) need
+  const bool can_split = part && (!deferred || (M * N) % 4 == 0) && aligned(part, 16) && aligned(y, 16) &&
+                         (!res || aligned(res, 16));
+  LinPlan plan = linear_plan(M, N, K, group, can_split ? std::min<size_t>(part_bytes, size_t{1} << 33) : 0,
+                             deferred != nullptr);
   const int ov = debug_override(Q4_DBG_LINEAR_TILE);
   if (ov >= 0 && ov < kNumLinWs) plan = LinPlan{ov, {1, 0}};
   const int ti = plan.tile, S = plan.split.n_split;
@@ -1119,10 +1134,9 @@ int q4_linear_planes(const uint16_t* xh, const uint16_t* xl, int64_t M, const in
     *deferred = S;
     return Q4_OK;
   }
-  const int64_t n4 = M * N / 4;
-  hipLaunchKernelGGL(linear_reduce_kernel, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, st,
+  hipLaunchKernelGGL(linear_reduce_kernel, dim3(static_cast<unsigned>((M * N + 1023) / 1024)), dim3(256), 0, st,
                      reinterpret_cast<const float4*>(part), reinterpret_cast<const float4*>(res),
-                     reinterpret_cast<float4*>(y), n4, S);
+                     reinterpret_cast<float4*>(y), M * N, S);
   return launch_status();
 }
 
@@ -1159,8 +1173,12 @@ int q4_linear_planes_swiglu(const uint16_t* xh, const uint16_t* xl, int64_t M, c
 int q4_linear_ws_launch(const float* x, int64_t M, const int32_t* qw, const uint16_t* sc, float* y, const float* res,
                         int64_t N, int64_t K, int group, void* ws, size_t ws_bytes, hipStream_t st) {
   // the pipelined kernel indexes groups by shifts: other group sizes take the workspace-free kernel,
-  // as do few rows (Q4_DBG_LINEAR_TILE set: the pipelined kernel)
-  if ((group & (group - 1)) || (q4_rows_takes(M, K) && !debug_set(Q4_DBG_LINEAR_TILE)))
+  // as do few rows, and K of at most two stages while its 64x64 tiles run at once, where the launch that
+  // splits x costs more than it gives: 250x3560x128 7.8 -> 6.2 us, 33x256x128 6.4 -> 5.5 (two rounds of
+  // tiles, 700x3560x128: 12.7 | 14.9); K 384 is past the line, 250x3560x384 10.3 | 11.4
+  // (Q4_DBG_LINEAR_TILE set: the pipelined kernel)
+  const bool short_k = K <= 128 && ((M + 63) / 64) * ((N + 63) / 64) <= 512;
+  if ((group & (group - 1)) || ((short_k || q4_rows_takes(M, K)) && !debug_set(Q4_DBG_LINEAR_TILE)))
     return q4_linear_launch(x, M, qw, sc, y, res, N, K, group, -1, st);
   uint16_t* xh = static_cast<uint16_t*>(ws);
   uint16_t* xl = xh + M * K;
