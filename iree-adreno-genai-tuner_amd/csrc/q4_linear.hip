@@ -1082,12 +1082,12 @@ LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes,
   return best;
 }
 
-// The rule: chunks of at most 256 rows whose partials the next kernel adds (a model step) take
-// linear_split_plan where it splits; everything else the cheapest tile.
-LinPlan linear_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool deferred) {
+// The rule: a model step's chunks of at most 256 rows (whose partials the next kernel adds, or, with the same
+// bits, linear_reduce_kernel) take linear_split_plan where it splits; everything else the cheapest tile.
+LinPlan linear_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool step) {
   const LinearSplit sp = linear_split_plan(M, N, K, group);
-  if (deferred && sp.n_split > 1 && part_bytes >= linear_split_part_bytes(M, N, K, group)) return LinPlan{kSplitTile, sp};
-  return tile_plan(M, N, K, group, deferred && M <= 256 ? 0 : part_bytes, !deferred);
+  if (step && sp.n_split > 1 && part_bytes >= linear_split_part_bytes(M, N, K, group)) return LinPlan{kSplitTile, sp};
+  return tile_plan(M, N, K, group, step && M <= 256 ? 0 : part_bytes, !step);
 }
 }  // namespace
 
@@ -1100,7 +1100,8 @@ size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
 
 // The pipelined GEMM on x given as fp16 (hi, lo) planes (store_x_planes layout, [M, K] each);
 // power-of-two groups only. linear_plan picks the tile and, with a partial buffer `part` that holds it,
-// the K split, whose partials linear_reduce_kernel adds. Q4_DBG_LINEAR_TILE overrides (no K split).
+// the K split, whose partials linear_reduce_kernel adds. Q4_DBG_LINEAR_TILE overrides (no K split). `t16`
+// (its tiles may be null) marks a projection of the model step, the only caller that has one.
 int q4_linear_planes(const uint16_t* xh, const uint16_t* xl, int64_t M, const int32_t* qw, const uint16_t* sc,
                      float* y, const float* res, int64_t N, int64_t K, int group, hipStream_t st, float* part,
                      size_t part_bytes, int* deferred, const T16Src* t16) {
@@ -1111,7 +1112,7 @@ int q4_linear_planes(const uint16_t* xh, const uint16_t* xl, int64_t M, const in
   const bool can_split = part && (!deferred || (M * N) % 4 == 0) && aligned(part, 16) && aligned(y, 16) &&
                          (!res || aligned(res, 16));
   LinPlan plan = linear_plan(M, N, K, group, can_split ? std::min<size_t>(part_bytes, size_t{1} << 33) : 0,
-                             deferred != nullptr);
+                             t16 != nullptr);
   const int ov = debug_override(Q4_DBG_LINEAR_TILE);
   if (ov >= 0 && ov < kNumLinWs) plan = LinPlan{ov, {1, 0}};
   const int ti = plan.tile, S = plan.split.n_split;
