@@ -187,7 +187,13 @@ int step_impl(const q4llm_model* m, const int32_t* tokens, int C, const int32_t*
   // Prefill with a power-of-two group: the norms, the attention merge and SwiGLU write their results
   // straight as the fp16 (hi, lo) planes the following projection reads (in the lin workspace).
   const int kmax = std::max(D, std::max(nq_w, m->inter));
-  const bool planes = C > 1 && (m->group & (m->group - 1)) == 0 && linear_fits(D, m->group) &&
+  // A few rows take the other path, whose projections are one launch each and read fp32 rows: what the tiled
+  // path fills with padding and K splits costs more there. Measured (6 layers of dim 3072, inter 8192, group
+  // 128 | 4 layers of dim 1024, inter 3072, group 32; tiled -> this, us): C = 2 527 -> 410 | 315 -> 183, C = 8
+  // 542 -> 462 | 325 -> 203, C = 16 566 -> 533 | 337 -> 219. From 17 rows on while C dim <= 65536 (inter 4096:
+  // C = 17 535 -> 509, C = 24 560 -> 558, C = 32 592 -> 605; dim 1024: C = 32 365 -> 262).
+  const bool few_rows = q4::q4_rows_takes(C, kmax) && (C <= 16 || static_cast<int64_t>(C) * D <= 65536);
+  const bool planes = C > 1 && !few_rows && (m->group & (m->group - 1)) == 0 && linear_fits(D, m->group) &&
                       linear_fits(nq_w, m->group) && linear_fits(m->inter, m->group);
   uint16_t* xh = static_cast<uint16_t*>(lin_ws);
   uint16_t* xl = xh + static_cast<size_t>(C) * kmax;

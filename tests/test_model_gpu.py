@@ -206,6 +206,25 @@ def test_prefill_chunk128_k_split_paths_vs_oracle(dev, kernel_override):
         assert (l_o.cpu() - r_l).abs().max().item() <= tol(r_l), s0
 
 
+@pytest.mark.parametrize("chunk", [2, 15, 16, 17, 32, 33])
+@pytest.mark.parametrize("cfg_kw", [dict(), dict(hidden_size=512, intermediate_size=4160), dict(hidden_size=2048)])
+def test_prefill_few_rows_vs_oracle(dev, cfg_kw, chunk):
+    """Chunks on both sides of the line between the few-rows projections and the tiled ones (16 rows; 32
+    rows of dim up to 2048; an inter size past 4096 tiles from 17 rows on): two chunks, the second reading
+    the first's caches, next token and logits against the oracle."""
+    cfg = dict(synth.TINY, num_hidden_layers=2, **cfg_kw)
+    ours, ref = build_pair(cfg, 32, 128)
+    prompt = synth.prompt_ids(2 * chunk, cfg["vocab_size"], seed=chunk)
+    c_ours, c_ref = ours.new_caches(), ref.new_caches()
+    for s0 in (0, chunk):
+        toks = torch.tensor([prompt[s0:s0 + chunk]], dtype=torch.int32)
+        start, last = torch.tensor([s0], dtype=torch.int32), torch.tensor([chunk - 1], dtype=torch.int32)
+        n_o, l_o = ours.step(toks, start, last, c_ours, 128)
+        r_n, r_l = ref.step(toks, start, last, c_ref, 128)
+        assert int(n_o.item()) == int(r_n.item()), s0
+        assert (l_o.cpu() - r_l).abs().max().item() <= tol(r_l), s0
+
+
 @pytest.mark.parametrize("cfg_kw,chunk", [
     # qkv and o: 4 partials each; down: 128 (past the 12 loaded with the row: the tail loop); gate/up: 2
     (dict(intermediate_size=8192), 128),
