@@ -73,13 +73,13 @@ struct LinearSplit {
   int n_split, nk_split;
 };
 LinearSplit linear_split_plan(int64_t M, int64_t N, int64_t K, int group);
-// bytes of K-split partials q4_linear_planes uses for this shape (0: it takes no K split)
+// bytes of K-split partials that a model step holds for this shape (0: no split past 256 rows)
 size_t linear_split_part_bytes(int64_t M, int64_t N, int64_t K, int group);
-// the same for q4_linear_ws, which may split K past 256 rows too
+// with which q4_linear_ws takes its fastest plan, past 256 rows too
 size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group);
 
-// q4_linear_ws's GEMM on given planes (power-of-two group); with `part` (at least
-// linear_split_part_bytes, 16-byte aligned) it may split K and reduce the partials in a second kernel.
+// q4_linear_ws's GEMM on given planes (power-of-two group); with `part` (part_bytes, 16-byte aligned) it
+// may split K and reduce the partials in a second kernel.
 // With `deferred` not null, a K split leaves its partials in `part` unreduced and sets *deferred to the
 // number of splits (0 when the result went to y); the caller's next kernel then completes y.
 // The decode T16 copy of the same weight (q4_t16_pack: tiles, scales, and the pairing and head size it

@@ -999,8 +999,9 @@ int planes_args(const uint16_t* xh, const uint16_t* xl, int64_t M, const int32_t
 }
 }  // namespace
 
-// K split of the 64x256 tile (kSplitTile) for a chunk of M <= 256 rows whose tiles alone would leave
-// CUs idle: about 256 / tiles splits, each a whole number of groups (64-k stages, at least one group).
+// What sizes the partials of a chunk of M <= 256 rows: the K split of the 64x256 tile (kSplitTile) that fills
+// the chip, about 256 / tiles splits, each a whole number of groups (64-k stages, at least one group).
+// tile_plan below chooses the split that runs, within that space.
 LinearSplit linear_split_plan(int64_t M, int64_t N, int64_t K, int group) {
   LinearSplit p{1, 0};
   if (M <= 0 || M > 256 || K % 64 || group <= 0) return p;
@@ -1060,7 +1061,8 @@ double tile_time(int ti, int64_t wgs, int64_t steps, int group) {
 // Against the 64x64 and 32x64 tiles that ran all of these before (us, with the x split): 512x5120x3072
 // 78.8 -> 52.4, 512x16384x3072 197 -> 100 (group 32: 241 -> 135), 1024x5120x3072 127 -> 83, 1024x16384x3072
 // 375 -> 190. Against a split of every M <= 256 into about 256 workgroups of 64x256 (linear_split_plan), short
-// K: 250x3560x384 17.6 -> 10.3, 250x3072x1024 21.0 -> 16.0, 100x8192x1024 21.5 -> 15.5, 33x16384x640 16.5 -> 11.6.
+// K: 250x3560x384 17.6 -> 10.3, 250x3072x1024 21.0 -> 16.0, 100x8192x1024 21.5 -> 15.5, 33x16384x640 16.5 -> 11.6;
+// in a step (4 layers, group 64, 87 rows, dim 512, inter 7296) 455 -> 352, none changed at dim 3072, group 128.
 LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool reduce) {
   const int64_t nk = K / 64, gst = group > 64 ? group / 64 : 1;
   LinPlan best{kSmallTile, {1, 0}};
@@ -1082,24 +1084,17 @@ LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes,
   return best;
 }
 
-// The rule: a model step's chunks of at most 256 rows (whose partials the next kernel adds, or, with the same
-// bits, linear_reduce_kernel) take linear_split_plan where it splits; everything else the cheapest tile.
-LinPlan linear_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool step) {
-  const LinearSplit sp = linear_split_plan(M, N, K, group);
-  if (step && sp.n_split > 1 && part_bytes >= linear_split_part_bytes(M, N, K, group)) return LinPlan{kSplitTile, sp};
-  return tile_plan(M, N, K, group, step && M <= 256 ? 0 : part_bytes, !step);
-}
 }  // namespace
 
 // Bytes of partials with which q4_linear_planes takes its fastest plan, outside the model step too
-// (there linear_split_part_bytes: no split past 256 rows).
+// (there linear_split_part_bytes).
 size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
   return std::max(linear_split_part_bytes(M, N, K, group),
                   tile_plan(M, N, K, group, SIZE_MAX, true).part_bytes(M, N));
 }
 
 // The pipelined GEMM on x given as fp16 (hi, lo) planes (store_x_planes layout, [M, K] each);
-// power-of-two groups only. linear_plan picks the tile and, with a partial buffer `part` that holds it,
+// power-of-two groups only. tile_plan picks the tile and, with a partial buffer `part` that holds it,
 // the K split, whose partials linear_reduce_kernel adds. Q4_DBG_LINEAR_TILE overrides (no K split). `t16`
 // (its tiles may be null) marks a projection of the model step, the only caller that has one.
 int q4_linear_planes(const uint16_t* xh, const uint16_t* xl, int64_t M, const int32_t* qw, const uint16_t* sc,
@@ -1111,8 +1106,7 @@ int q4_linear_planes(const uint16_t* xh, const uint16_t* xl, int64_t M, const in
   // what the partials and linear_reduce_kernel (a caller's next kernel: whole float4s too) need
   const bool can_split = part && (!deferred || (M * N) % 4 == 0) && aligned(part, 16) && aligned(y, 16) &&
                          (!res || aligned(res, 16));
-  LinPlan plan = linear_plan(M, N, K, group, can_split ? std::min<size_t>(part_bytes, size_t{1} << 33) : 0,
-                             t16 != nullptr);
+  LinPlan plan = tile_plan(M, N, K, group, can_split ? std::min<size_t>(part_bytes, size_t{1} << 33) : 0, !t16);
   const int ov = debug_override(Q4_DBG_LINEAR_TILE);
   if (ov >= 0 && ov < kNumLinWs) plan = LinPlan{ov, {1, 0}};
   const int ti = plan.tile, S = plan.split.n_split;
