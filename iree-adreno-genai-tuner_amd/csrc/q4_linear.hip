@@ -987,14 +987,15 @@ int q4_linear_ws_tile_info(int i, int* out) {
 namespace {
 // What the pipelined GEMM's index arithmetic assumes: every 64-k stage lies in whole groups of a
 // power of two >= 32 (at most two scale slots per stage, groups found by shifts), K a multiple of
-// 64, and 32-bit element offsets.
+// 64, 32-bit element offsets, and scales that start on a whole word (they are loaded by aligned words: a
+// row slice of a weight with an odd number of groups does not).
 int planes_args(const uint16_t* xh, const uint16_t* xl, int64_t M, const int32_t* qw, const uint16_t* sc, int64_t N,
                 int64_t K, int group) {
   if (!xh || !xl || !qw || !sc) return Q4_ERR_NULL;
   if (M <= 0 || N <= 0 || K <= 0 || group < 32 || (group & (group - 1)) || K % 64 || K % group) return Q4_ERR_SHAPE;
   if (M * K * 4 >= (int64_t{1} << 31) || N * (K / 2) >= (int64_t{1} << 31) || M > INT32_MAX || N > INT32_MAX)
     return Q4_ERR_SHAPE;
-  if (!aligned(xh, 16) || !aligned(xl, 16) || !aligned(qw, 16)) return Q4_ERR_ALIGN;
+  if (!aligned(xh, 16) || !aligned(xl, 16) || !aligned(qw, 16) || !aligned(sc, 4)) return Q4_ERR_ALIGN;
   return Q4_OK;
 }
 }  // namespace
@@ -1167,13 +1168,13 @@ int q4_linear_planes_swiglu(const uint16_t* xh, const uint16_t* xl, int64_t M, c
 // the K-split partials.
 int q4_linear_ws_launch(const float* x, int64_t M, const int32_t* qw, const uint16_t* sc, float* y, const float* res,
                         int64_t N, int64_t K, int group, void* ws, size_t ws_bytes, hipStream_t st) {
-  // the pipelined kernel indexes groups by shifts: other group sizes take the workspace-free kernel,
-  // as do few rows, and K of at most two stages while its 64x64 tiles run at once, where the launch that
+  // the pipelined kernel indexes groups by shifts and loads scales by words (planes_args): other group sizes
+  // and scales take the workspace-free kernel, as do few rows, and K of at most two stages while its 64x64 tiles run at once, where the launch that
   // splits x costs more than it gives: 250x3560x128 7.8 -> 6.2 us, 33x256x128 6.4 -> 5.5 (two rounds of
   // tiles, 700x3560x128: 12.7 | 14.9); K 384 is past the line, 250x3560x384 10.3 | 11.4
   // (Q4_DBG_LINEAR_TILE set: the pipelined kernel)
   const bool short_k = K <= 128 && ((M + 63) / 64) * ((N + 63) / 64) <= 512;
-  if ((group & (group - 1)) || ((short_k || q4_rows_takes(M, K)) && !debug_set(Q4_DBG_LINEAR_TILE)))
+  if ((group & (group - 1)) || !aligned(sc, 4) || ((short_k || q4_rows_takes(M, K)) && !debug_set(Q4_DBG_LINEAR_TILE)))
     return q4_linear_launch(x, M, qw, sc, y, res, N, K, group, -1, st);
   uint16_t* xh = static_cast<uint16_t*>(ws);
   uint16_t* xl = xh + M * K;

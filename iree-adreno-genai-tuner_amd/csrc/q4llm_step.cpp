@@ -91,6 +91,16 @@ int layout_for(const q4llm_model* m, int C, int L, Layout* lo) {
   return Q4_OK;
 }
 
+// The pipelined prefill GEMM loads group scales by whole words.
+bool scales_on_words(const q4llm_model* m) {
+  for (int i = 0; i < m->n_layers; ++i) {
+    const q4llm_layer& l = m->layers[i];
+    for (const uint16_t* s : {l.wqkv_s, l.wo_s, l.wgu_s, l.wdown_s})
+      if (!q4::aligned(s, 4)) return false;
+  }
+  return true;
+}
+
 int check_model(const q4llm_model* m) {
   if (!m || !m->layers || !m->embed_q || !m->embed_s || !m->ln_f || !m->cos_t || !m->sin_t) return Q4_ERR_NULL;
   if (m->dim <= 0 || m->n_layers <= 0 || m->n_heads <= 0 || m->n_kv <= 0 || m->head_dim <= 0 || m->inter <= 0 ||
@@ -194,7 +204,7 @@ int step_impl(const q4llm_model* m, const int32_t* tokens, int C, const int32_t*
   // C = 17 535 -> 509, C = 24 560 -> 558, C = 32 592 -> 605; dim 1024: C = 32 365 -> 262).
   const bool few_rows = q4::q4_rows_takes(C, kmax) && (C <= 16 || static_cast<int64_t>(C) * D <= 65536);
   const bool planes = C > 1 && !few_rows && (m->group & (m->group - 1)) == 0 && linear_fits(D, m->group) &&
-                      linear_fits(nq_w, m->group) && linear_fits(m->inter, m->group);
+                      linear_fits(nq_w, m->group) && linear_fits(m->inter, m->group) && scales_on_words(m);
   uint16_t* xh = static_cast<uint16_t*>(lin_ws);
   uint16_t* xl = xh + static_cast<size_t>(C) * kmax;
   const hipStream_t st = static_cast<hipStream_t>(stream);

@@ -92,6 +92,23 @@ def test_linear_many_rows(dev, M, N, K, group):
         assert ((h.cpu().double() - ref).abs() <= bound).all(), split
 
 
+@pytest.mark.parametrize("M,N,K,group", [(33, 200, 384, 128), (100, 257, 320, 64), (300, 515, 1152, 128), (9, 40, 384, 128),
+                                         (40, 96, 96 * 2, 32 * 3)])
+def test_linear_scales_off_a_word(dev, M, N, K, group):
+    """Rows 1.. of a weight with an odd number of groups: its scales start between two words, which the
+    kernel that loads them by words must not take."""
+    x, qw, sc, res, ref, bound = linear_case(dev, M, N + 1, K, group, M + N)
+    ref, bound, qw, sc, res = ref[:, 1:], bound[:, 1:], qw[1:], sc[1:], res[:, 1:].contiguous()
+    if K // group % 2:
+        assert sc.data_ptr() % 4 == 2
+    for fn in (ops.q4_linear, ops.q4_linear_ws):
+        y = fn(x, qw, sc, group, residual=res)
+        assert ((y.cpu().double() - ref).abs() <= bound).all(), fn
+        y = torch.full((M, N), float("nan"), device=dev)
+        fn(x, qw, sc, group, out=y)
+        assert ((y.cpu().double() - (ref - res.cpu().double())).abs() <= bound).all(), fn
+
+
 def attn_ref64(q, kc, vc, start, scale):
     C, nq, hd = q.shape
     n, nkv = min(start + C, kc.shape[0]), kc.shape[1]

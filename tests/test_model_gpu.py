@@ -283,6 +283,27 @@ def test_prefill_t16_source_matches_reference_layout(dev, kernel_override, chunk
     assert (l_t.cpu() - r_l).abs().max().item() <= tol(r_l)
 
 
+def test_prefill_scales_off_a_word_vs_oracle(dev, kernel_override):
+    """A model whose group scales start between two words (a C caller's own buffers): the prefill takes the
+    kernels that read them one by one; next token and logits against the oracle."""
+    ours, ref = build_pair(dict(synth.TINY, num_hidden_layers=2), 32, 128)
+    kernel_override("prefill_ref_layout", 1)
+    for ly in ours.layers:
+        for lin in (ly.wqkv, ly.wo, ly.wgu, ly.wdown):
+            buf = torch.empty(lin.scales.numel() + 1, dtype=torch.float16, device=dev)
+            buf[1:].copy_(lin.scales.reshape(-1))
+            lin.scales = torch.nn.Parameter(buf[1:].view(lin.scales.shape), requires_grad=False)
+            assert lin.scales.data_ptr() % 4 == 2
+    ours._desc = None
+    prompt = synth.prompt_ids(100, 1024, seed=2)
+    toks = torch.tensor([prompt], dtype=torch.int32)
+    start, last = torch.tensor([0], dtype=torch.int32), torch.tensor([99], dtype=torch.int32)
+    n_o, l_o = ours.step(toks, start, last, ours.new_caches(), 128)
+    r_n, r_l = ref.step(toks, start, last, ref.new_caches(), 128)
+    assert int(n_o.item()) == int(r_n.item())
+    assert (l_o.cpu() - r_l).abs().max().item() <= tol(r_l)
+
+
 def test_group16_step_and_generation_vs_oracle(dev):
     """group 16 (legal in the reference: group % 8 == 0, llama_q4.py:31): the matrix-core prefill GEMM
     takes only groups of 32 * 2^j, so prefill runs one GEMV per row; decode takes the generic GEMV
