@@ -231,10 +231,10 @@ int gemm_f16_nt_ws_bytes(int64_t M, int64_t N, int64_t K, size_t* bytes);
  * alone leave CUs idle, K is split over several workgroups per tile, each writing an fp32 partial
  * into the workspace, and a second launch adds the partials in a fixed order and writes C, so the
  * result does not depend on timing. Same argument rules and result tolerance as gemm_f16_nt;
- * Q4_ERR_WORKSPACE when the workspace is missing or too small (from M = 512 on a smaller one, or none,
- * is taken: the best plan that fits it runs). Replaces the same call of the
- * reference's harness (gemm/harness/vk_gemm_bench.c dispatch of one NT problem) where the caller
- * can hold a workspace. */
+ * Q4_ERR_WORKSPACE when the workspace is missing or too small; problems of M >= 512 and at least
+ * 4 GFLOP (2 M N K >= 4e9) also take a smaller one, or none, and run the best plan that fits it.
+ * Replaces the same call of the reference's harness (gemm/harness/vk_gemm_bench.c dispatch of one NT
+ * problem) where the caller can hold a workspace. */
 int gemm_f16_nt_ws(const uint16_t* A, const uint16_t* B, uint16_t* C, int64_t M, int64_t N, int64_t K,
                    int64_t lda, int64_t ldb, int64_t ldc, void* workspace, size_t workspace_bytes,
                    void* stream);

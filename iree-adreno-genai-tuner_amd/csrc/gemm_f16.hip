@@ -595,9 +595,9 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, size_t part_bytes) {
   return best;
 }
 
-// Whether gemm_f16_nt_ws takes this workspace: all that the split by size alone needs (latency-bound
-// problems and M < 512; none from there on), or all that the plan asks for. With less than the plan asks
-// for, the call runs the best plan that fits.
+// Whether gemm_f16_nt_ws takes this workspace: all that the split by size alone needs (problems under
+// 4 GFLOP at any M, and M < 512; none for the rest), or all that the plan asks for. With less than the plan
+// asks for, the call runs the best plan that fits.
 bool gemm_workspace_ok(int64_t M, int64_t N, int64_t K, const void* ws, size_t ws_bytes) {
   if (M == 1) return true;
   const bool usable = ws && aligned(ws, 16);

@@ -259,7 +259,7 @@ def gemm_f16_nt_ws_bytes(m, n, k) -> int:
 def gemm_f16_nt_ws(a, b, out=None, workspace=None):
     """gemm_f16_nt with a device workspace (uint8, >= gemm_f16_nt_ws_bytes): K split over several
     workgroups per output tile where the tiles alone leave CUs idle, partials added in a fixed order.
-    A workspace is allocated when none is given."""
+    A workspace is allocated when none is given; without memory for it gemm_f16_nt runs."""
     if out is None and workspace is not None:
         c = _gemm(a, b, workspace)
         if c is not None:
@@ -278,10 +278,10 @@ def gemm_f16_nt_ws(a, b, out=None, workspace=None):
     if workspace is None:
         try:
             workspace = torch.empty(max(gemm_f16_nt_ws_bytes(m, n, k), 16), dtype=torch.uint8, device=a.device)
-        except torch.OutOfMemoryError:
-            if m < 512:
-                raise
-            workspace = torch.empty(16, dtype=torch.uint8, device=a.device)  # from 512 rows on, any size is taken
+        except torch.OutOfMemoryError:  # the form that needs none
+            LIB.call("gemm_f16_nt", ptr(a), ptr(b), ptr(out), m, n, k, a.stride(0), b.stride(0), out.stride(0),
+                     stream_of(a.device))
+            return out
     _need(workspace, "workspace", torch.uint8, None)
     LIB.call("gemm_f16_nt_ws", ptr(a), ptr(b), ptr(out), m, n, k, a.stride(0), b.stride(0), out.stride(0),
              ptr(workspace), workspace.numel(), stream_of(a.device))

@@ -177,6 +177,35 @@ def test_gemm_plan_and_workspace_sizes(dev, M, N, K):
     check(ops.gemm_f16_nt_ws(a, b), "its own workspace")
 
 
+@pytest.mark.parametrize("M,N,K", [(512, 1024, 1024), (4096, 64, 4096), (1000, 256, 2048), (511, 1024, 4096), (256, 3072, 8192),
+                                   (512, 3072, 8192), (513, 1024, 4096)])
+def test_gemm_workspace_contract(dev, monkeypatch, M, N, K):
+    """Which workspaces gemm_f16_nt_ws takes, on both sides of 512 rows and 4 GFLOP: the size it asks for and
+    more always; less, or none, only from both lines on. Without memory for a workspace the wrapper runs
+    the form that needs none."""
+    a, b = torch.ones(M, K, device=dev).half(), torch.ones(N, K, device=dev).half() / 64
+    need = ops.gemm_f16_nt_ws_bytes(M, N, K)
+    f = LIB.raw("gemm_f16_nt_ws")
+    st = torch.cuda.current_stream(dev).cuda_stream
+    lenient = M >= 512 and 2 * M * N * K >= 4e9
+    assert need > 0
+    for nbytes in (0, need // 2, need - 16, need, need + 64):
+        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
+        c = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+        rc = f(ops.ptr(a), ops.ptr(b), ops.ptr(c), M, N, K, K, K, N, ops.ptr(ws) if nbytes else None, nbytes, st)
+        assert rc == (0 if nbytes >= need or lenient else -5), nbytes
+        assert rc != 0 or (c == K / 64).all()
+    empty = torch.empty
+
+    def no_workspace(*args, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no memory")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_workspace)
+    assert (ops.gemm_f16_nt_ws(a, b) == K / 64).all()
+
+
 def test_native_calls_match_python_wrappers(dev, monkeypatch):
     """The native calls and the Python wrappers they stand in for give the same bits and the same errors,
     on the current stream; operands the native code leaves alone (views that need a copy, an `out`, other
