@@ -48,15 +48,25 @@ def _compile(src: pathlib.Path, obj: pathlib.Path) -> None:
         print(err, file=sys.stderr)
 
 
-def build_torch_module() -> pathlib.Path:
-    """lib/_q4torch.so (csrc/q4_torch.cpp): host code over libq4llm.so and the installed torch's headers."""
-    torch_dir = pathlib.Path(importlib.util.find_spec("torch").submodule_search_locations[0])
+def build_torch_module():
+    """lib/_q4torch.so (csrc/q4_torch.cpp): host code over libq4llm.so and the installed torch's headers.
+    Without a torch for ROCm, its headers or Python's there is nothing to build it for: returns None, and a
+    module of an earlier build goes (q4llm/ops.py then makes the same calls through ctypes)."""
     out = LIB / "_q4torch.so"
     tmp = LIB / "_q4torch.so.tmp"
+    spec = importlib.util.find_spec("torch")
+    torch_dir = pathlib.Path(spec.submodule_search_locations[0]) if spec else None
+    py_inc = pathlib.Path(sysconfig.get_paths()["include"])
+    needs = [torch_dir / "include" / h for h in ("torch/csrc/autograd/python_variable.h", "c10/hip/HIPStream.h")] if spec else []
+    missing = [str(h) for h in [*needs, py_inc / "Python.h"] if not h.exists()] + ([] if spec else ["torch"])
+    if missing:
+        out.unlink(missing_ok=True)
+        print(f"torch module not built, not found: {', '.join(missing)}", file=sys.stderr)
+        return None
     inc = torch_dir / "include"
     cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__",
            "-DUSE_ROCM", "-isystem", str(inc), "-isystem", str(inc / "torch/csrc/api/include"), "-isystem",
-           "/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", f"-I{ROOT / 'include'}",
+           "/opt/rocm/include", f"-I{py_inc}", f"-I{ROOT / 'include'}",
            str(CSRC / "q4_torch.cpp"), "-o", str(tmp), f"-L{LIB}", "-lq4llm", f"-L{torch_dir / 'lib'}", "-ltorch_python",
            "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
     r = subprocess.run(cmd, capture_output=True, text=True)
