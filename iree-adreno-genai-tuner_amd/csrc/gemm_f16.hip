@@ -452,19 +452,20 @@ struct TileCfg {
   int bm, bn, wgm, wgn, nst, bk;
   bool sp = false;  // software-pipelined substeps (gemm_f16_nt_kernel<..., true>)
 };
-// Explicit CDNA4 tile list (index stable for gemm_f16_nt_cfg / the Q4_DBG_GEMM_TILE override).
+// Explicit CDNA4 tile list. An entry keeps its index (gemm_f16_nt_cfg and the Q4_DBG_GEMM_TILE override select
+// by it): a new one takes the place of a removed one (3 and 4, once 64x96 and 128x64) or the end.
 constexpr TileCfg kTiles[] = {
     {256, 256, 2, 4, 2, 64},        // 0: 8 waves of 128x64, 2 stages of K 64 (128 KB LDS)
     {128, 128, 2, 2, 2, 64},        // 1: 4 waves of 64x64, 2 stages (64 KB, two workgroups per CU)
-    {128, 128, 2, 2, 4, 64, true},  // 2: 4 waves of 64x64, 4 stages (128 KB), pipelined (entry 5 with one wave per
+    {128, 128, 2, 2, 4, 64, true},  // 2: 4 waves of 64x64, 4 stages (128 KB), pipelined (entry 3 with one wave per
                                     //    SIMD: for sweeps, the rule never takes it)
-    {64, 64, 2, 2, 4, 64},          // 3: 4 waves of 32x32, 4 stages (64 KB, two workgroups per CU)
-    {128, 160, 2, 5, 4, 64, true},  // 4: 10 waves of 64x32, 4 stages (145 KB), pipelined
-    {128, 128, 4, 2, 4, 64, true},  // 5: 8 waves of 32x64, 4 stages (128 KB), pipelined
-    {256, 128, 4, 2, 3, 64, true},  // 6: 8 waves of 64x64, 3 stages (144 KB), pipelined
+    {128, 128, 4, 2, 4, 64, true},  // 3: 8 waves of 32x64, 4 stages (128 KB), pipelined
+    {256, 128, 4, 2, 3, 64, true},  // 4: 8 waves of 64x64, 3 stages (144 KB), pipelined
+    {64, 64, 2, 2, 4, 64},          // 5: 4 waves of 32x32, 4 stages (64 KB, two workgroups per CU)
+    {128, 160, 2, 5, 4, 64, true},  // 6: 10 waves of 64x32, 4 stages (145 KB), pipelined
     {64, 128, 2, 4, 4, 64, true},   // 7: 8 waves of 32x32, 4 stages (96 KB), pipelined
 };
-constexpr int kSmallEntry = 3, kWideEntry = 2;  // the 64x64 tile; the 128x128 one that K splits are sized by below
+constexpr int kSmallEntry = 5, kWideEntry = 2;  // the 64x64 tile; the 128x128 one that K splits are sized by below
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
 using GemmFn = void (*)(const uint16_t*, const uint16_t*, uint16_t*, int, int, int, int, int, int, int, int, int, int,
@@ -546,8 +547,8 @@ double tile_time(int ti, int64_t wgs, int64_t steps) {
     int cap;
   };
   constexpr Rate kRates[kNumTiles] = {{8.9, 1.6, 1.346, 0.036, 256}, {5.7, 3.4, 0.575, 0.182, 512}, {0, 0, 0, 0, 0},
-                                      {3.2, 1.5, 0.322, 0.061, 512}, {5.1, 2.1, 0.568, 0.110, 256},
                                       {4.5, 2.6, 0.443, 0.086, 256}, {6.2, 1.5, 0.740, 0.147, 256},
+                                      {3.2, 1.5, 0.322, 0.061, 512}, {5.1, 2.1, 0.568, 0.110, 256},
                                       {3.5, 2.0, 0.354, 0.041, 256}};
   const Rate& r = kRates[ti];
   const int64_t full = wgs / r.cap, rest = wgs % r.cap;

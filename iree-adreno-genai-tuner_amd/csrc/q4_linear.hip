@@ -895,18 +895,19 @@ struct LinWsTile {
   int bm, bn, wm, wn, nst, ks;
   bool pipe;
 };
-// Explicit tile list (index stable for Q4_DBG_LINEAR_TILE sweeps): the entries the rules below pick. Swept
-// and removed (slower on every 3B prefill shape at M = 128, 256 and 1024): 4-wave 64x64, 32x64 and
-// 64x128 wave tiles on 128x128, 64x128, 128x64 and 64x256, 32x128 wave tiles (4 or 8 waves on 64x256,
-// 128x128, 128x256, 64x512), 64x64 waves on 128x256, k-split 2-wave and 64x64 / 128x64 / 32x96 /
-// 32x128 / 32x160 variants.
+// Explicit tile list: the entries the rules below pick. An entry keeps its index (the Q4_DBG_LINEAR_TILE override
+// selects by it): a new one takes the place of a removed one (0, once 64x64) or the end. Swept and removed
+// (slower on every 3B prefill shape at M = 128, 256 and 1024): 4-wave 64x64, 32x64 and 64x128 wave tiles on
+// 128x128, 64x128, 128x64 and 64x256, 32x128 wave tiles (4 or 8 waves on 64x256, 128x128, 128x256, 64x512),
+// 64x64 waves on 128x256 without the software pipeline, k-split 2-wave and 64x64 / 128x64 / 32x96 / 32x128 /
+// 32x160 variants.
 constexpr LinWsTile kLinWsTiles[] = {
-    {32, 64, 1, 2, 4, 2},          // 0: 4 waves: 2 tiles of 32x32, each k-split over 2 waves (52 KB)
-    {64, 256, 2, 4, 4, 1, true},   // 1: 8 waves of 32x64, software-pipelined: one workgroup per CU for
+    {128, 256, 2, 4, 3, 1, true},  // 0: 8 waves of 64x64, 3 stages (127 KB), software-pipelined: many rows
+    {32, 64, 1, 2, 4, 2},          // 1: 4 waves: 2 tiles of 32x32, each k-split over 2 waves (52 KB)
+    {64, 256, 2, 4, 4, 1, true},   // 2: 8 waves of 32x64, software-pipelined: one workgroup per CU for
                                    // 256-row chunks, and the K split
-    {128, 256, 2, 4, 3, 1, true},  // 2: 8 waves of 64x64, 3 stages (127 KB), software-pipelined: many rows
 };
-constexpr int kSmallTile = 0, kSplitTile = 1, kLargeTile = 2;  // kSplitTile: also the SwiGLU-epilogue tile
+constexpr int kLargeTile = 0, kSmallTile = 1, kSplitTile = 2;  // kSplitTile: also the SwiGLU-epilogue tile
 using LinWsFn = void (*)(const uint16_t*, const uint16_t*, const int32_t*, const uint16_t*, float*, const float*, int,
                          int, int, int, int, int, int, float*, int, int);
 template <int I>
@@ -926,7 +927,7 @@ constexpr size_t lin_ws_lds() {
   return LinWsCfg<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks>::kLds;
 }
 constexpr LinWsFn kLinWsFns[] = {lin_ws_fn<0>(), lin_ws_fn<1>(), lin_ws_fn<2>()};
-constexpr LinWsFn kLinWsT16Fns[] = {nullptr, lin_ws_t16_fn<0, kSplitTile>(), lin_ws_t16_fn<0, kLargeTile>()};
+constexpr LinWsFn kLinWsT16Fns[] = {lin_ws_t16_fn<0, kLargeTile>(), nullptr, lin_ws_t16_fn<0, kSplitTile>()};
 constexpr size_t kLinWsLds[] = {lin_ws_lds<0>(), lin_ws_lds<1>(), lin_ws_lds<2>()};
 static_assert(kLinWsTiles[kSplitTile].pipe && kLinWsTiles[kSplitTile].ks == 1 && kLinWsTiles[kLargeTile].pipe &&
                   kLinWsTiles[kLargeTile].ks == 1,
@@ -1046,8 +1047,8 @@ double tile_time(int ti, int64_t wgs, int64_t steps, int group) {
     double fixed, round, step, load;
     int cap;
   };
-  constexpr Rate kRates[2][3] = {{{5.7, 1.0, 0.352, 0.112, 768}, {7.2, 0, 0.801, 0.201, 256}, {8.7, 0, 1.318, 0.200, 256}},
-                                 {{5.7, 1.0, 0.397, 0.125, 768}, {7.3, 0, 1.258, 0.167, 256}, {8.7, 0, 2.030, 0.100, 256}}};
+  constexpr Rate kRates[2][3] = {{{8.7, 0, 1.318, 0.200, 256}, {5.7, 1.0, 0.352, 0.112, 768}, {7.2, 0, 0.801, 0.201, 256}},
+                                 {{8.7, 0, 2.030, 0.100, 256}, {5.7, 1.0, 0.397, 0.125, 768}, {7.3, 0, 1.258, 0.167, 256}}};
   const Rate& r = kRates[group >= 128 ? 0 : 1][ti];
   const int64_t full = wgs / r.cap, rest = wgs % r.cap;
   double us = r.fixed + static_cast<double>(full - (rest ? 0 : 1)) * r.round;
