@@ -75,7 +75,7 @@ struct LinearSplit {
 LinearSplit linear_split_plan(int64_t M, int64_t N, int64_t K, int group);
 // bytes of K-split partials that a model step holds for this shape (0: no split past 256 rows)
 size_t linear_split_part_bytes(int64_t M, int64_t N, int64_t K, int group);
-// with which q4_linear_ws takes its fastest plan, past 256 rows too
+// that q4_linear_ws writes on its fastest plan for this shape (0: no split)
 size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group);
 
 // q4_linear_ws's GEMM on given planes (power-of-two group); with `part` (part_bytes, 16-byte aligned) it

@@ -482,6 +482,20 @@ def test_linear_ws_entries_cover_once(idx):
         replay_linear_ws(cfg, 100, 3 * cfg[1] + 32, 512, group)
 
 
+@pytest.mark.parametrize("M,N,K,group,splits", [
+    (64, 256, 704, 64, 1), (33, 520, 1024, 256, 1), (256, 16384, 3072, 128, 1), (1024, 5120, 3072, 128, 1),  # no split
+    (16, 1408, 256, 32, 1), (7, 3072, 3072, 128, 1), (24, 3072, 3072, 128, 1), (250, 3560, 128, 128, 1),  # one launch
+    (40, 96, 192, 96, 1),  # a group that is no power of two: the workspace-free kernel
+    (64, 256, 2048, 64, 16), (70, 1408, 1536, 32, 12), (50, 520, 2048, 256, 8), (256, 5120, 3072, 128, 3), (100, 515, 3072, 32, 16)])
+def test_linear_ws_split_bytes_is_what_the_call_writes(M, N, K, group, splits):
+    """q4_linear_ws_split_bytes: the planes alone wherever the call adds no partials, else the planes (from a
+    256-byte boundary) and `splits` times M N fp32 partials (whole float4s): nothing more is allocated per call."""
+    from q4llm import ops
+    planes = 4 * M * K
+    part = splits * cdiv(M * N, 4) * 16 if splits > 1 else 0
+    assert ops.q4_linear_ws_split_bytes(M, N, K, group) == (cdiv(planes, 256) * 256 + part if part else planes)
+
+
 @pytest.mark.parametrize("bk", [64, 32])
 def test_gemm_swizzle_is_bank_conflict_free(bk):
     """An MFMA operand read takes 16 consecutive tile rows at one 16-byte chunk; gfx950's LDS serves
