@@ -65,6 +65,8 @@ int argmax_final_launch(const ArgBest* partials, int n, int32_t* out, int32_t* a
 // q4_linear for a few rows of x in one launch (q4_rows.hip), for the sizes q4_rows_takes; arguments
 // checked by the caller (K % 64 == 0, group % 32 == 0, M <= 32).
 bool q4_rows_takes(int64_t M, int64_t K);
+// whether it is also faster than the tiled path with a workspace
+bool q4_rows_wins(int64_t M, int64_t N, int64_t K, int group);
 int q4_rows_launch(const float* x, int64_t M, const int32_t* qw, const uint16_t* sc, float* y, const float* res,
                    int64_t N, int64_t K, int group, hipStream_t st);
 

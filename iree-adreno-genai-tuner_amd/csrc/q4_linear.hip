@@ -1089,18 +1089,20 @@ LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes,
 }  // namespace
 
 namespace {
-// Calls of q4_linear_ws that one launch without planes or partials serves better: a few rows, and K of at
-// most two stages while its 64x64 tiles run at once, where the launch that splits x costs more than it
+// Calls of q4_linear_ws that one launch without planes or partials serves better: a few rows (q4_rows_wins;
+// short of the partials that the tiles need, all that the kernel takes), and K of at most two stages while its 64x64 tiles run at once, where the launch that splits x costs more than it
 // gives: 250x3560x128 7.8 -> 6.2 us, 33x256x128 6.4 -> 5.5 (two rounds of tiles, 700x3560x128: 12.7 | 14.9);
 // K 384 is past the line, 250x3560x384 10.3 | 11.4.
-bool one_launch(int64_t M, int64_t N, int64_t K) {
-  return q4_rows_takes(M, K) || (K <= 128 && ((M + 63) / 64) * ((N + 63) / 64) <= 512);
+bool one_launch(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes) {
+  if (K <= 128 && ((M + 63) / 64) * ((N + 63) / 64) <= 512) return true;
+  return q4_rows_wins(M, N, K, group) ||
+         (q4_rows_takes(M, K) && part_bytes < tile_plan(M, N, K, group, SIZE_MAX, true).part_bytes(M, N));
 }
 }  // namespace
 
 // Bytes of partials with which q4_linear_ws takes its fastest plan (the model step: linear_split_part_bytes).
 size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
-  return one_launch(M, N, K) ? 0 : tile_plan(M, N, K, group, SIZE_MAX, true).part_bytes(M, N);
+  return one_launch(M, N, K, group, SIZE_MAX) ? 0 : tile_plan(M, N, K, group, SIZE_MAX, true).part_bytes(M, N);
 }
 
 // The pipelined GEMM on x given as fp16 (hi, lo) planes (store_x_planes layout, [M, K] each);
@@ -1179,7 +1181,8 @@ int q4_linear_ws_launch(const float* x, int64_t M, const int32_t* qw, const uint
                         int64_t N, int64_t K, int group, void* ws, size_t ws_bytes, hipStream_t st) {
   // the pipelined kernel indexes groups by shifts and loads scales by words (planes_args): other group sizes
   // and scales take the workspace-free kernels (Q4_DBG_LINEAR_TILE set: else the pipelined kernel)
-  if ((group & (group - 1)) || !aligned(sc, 4) || (one_launch(M, N, K) && !debug_set(Q4_DBG_LINEAR_TILE)))
+  const size_t planes = (static_cast<size_t>(M) * K * 4 + 255) / 256 * 256, room = ws_bytes > planes ? ws_bytes - planes : 0;
+  if ((group & (group - 1)) || !aligned(sc, 4) || (one_launch(M, N, K, group, room) && !debug_set(Q4_DBG_LINEAR_TILE)))
     return q4_linear_launch(x, M, qw, sc, y, res, N, K, group, -1, st);
   uint16_t* xh = static_cast<uint16_t*>(ws);
   uint16_t* xl = xh + M * K;
@@ -1187,9 +1190,8 @@ int q4_linear_ws_launch(const float* x, int64_t M, const int32_t* qw, const uint
   hipLaunchKernelGGL(split_x_kernel, dim3(static_cast<unsigned>((chunks + 255) / 256)), dim3(256), 0, st, x, xh, xl,
                      chunks);
   if (int e = launch_status()) return e;
-  const size_t planes = (static_cast<size_t>(M) * K * 4 + 255) / 256 * 256;
-  float* part = ws_bytes > planes ? reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + planes) : nullptr;
-  return q4_linear_planes(xh, xl, M, qw, sc, y, res, N, K, group, st, part, part ? ws_bytes - planes : 0);
+  float* part = room ? reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + planes) : nullptr;
+  return q4_linear_planes(xh, xl, M, qw, sc, y, res, N, K, group, st, part, room);
 }
 
 }  // namespace q4

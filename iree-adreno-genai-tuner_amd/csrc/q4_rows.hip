@@ -244,18 +244,38 @@ int rows_go(const float* x, int64_t M, const int32_t* qw, const uint16_t* sc, fl
 // (the one-tile-per-workgroup kernel before both: 70, 96, 186 and 48 us at every such M).
 bool q4_rows_takes(int64_t M, int64_t K) { return M <= 16 || (M <= 32 && K <= 4096); }
 
-// Columns per workgroup: about one workgroup per CU, so 16 up to 4096 columns, 32 up to 8192, else 64
+// Columns per workgroup / 16: about one workgroup per CU, so 16 columns up to 4096, 32 up to 8192, else 64
 // (M = 7: 5120 columns 8.6 us by 32 against 11.8 by 16, 16384 13.4 by 64 against 16.8 by 32).
+static int rows_nt(int64_t N) { return N <= 4096 ? 1 : N <= 8192 ? 2 : 4; }
+
+// Where a workspace makes the tiled path possible too, this kernel runs on its side of a line fitted to 2600
+// shapes of M 2-32, N 64-131072, K 256-28672 at groups 128 and 32 (graph replays over rotated weights; at most
+// 6% slower than the tiled path on any, and 0.5% off the faster one on average): M K below a limit that grows
+// with how full the chip is of workgroups, since the tiled path's K splits fill it at any N; more for groups
+// under 128, whose scales cost the tiles more; and up to a number of columns from where on both have work for
+// every CU and the tiles read x less often. This kernel | tiled path, group 128 (us): 16x4096x8192 21.3 | 22.7,
+// 16x4096x14336 34.3 | 28.5, 16x8192x14336 41.7 | 42.4, 12x8448x14336 54.1 | 47.4, 4x1536x28672 37.2 | 35.8,
+// 32x64x4096 18.4 | 13.9, 32x4096x4096 19.1 | 20.9, 7x65536x8192 121 | 153, 24x131072x2048 85.3 | 74.3.
+bool q4_rows_wins(int64_t M, int64_t N, int64_t K, int group) {
+  if (!q4_rows_takes(M, K)) return false;
+  const int nt = rows_nt(N);
+  const double fill = std::min(1.0, static_cast<double>((N + 16 * nt - 1) / (16 * nt)) / 256.0), f2 = fill * fill;
+  if (M <= 16) {
+    if (N > 49152 && (N > 65536 || K < (group < 128 ? 1024 : M <= 8 ? 3072 : 5120))) return false;
+    const double limit = (nt == 4 ? 65536.0 : 86016.0) + 81920.0 * nt * f2 * (nt == 1 ? 1.0 : nt == 2 ? fill : f2);
+    // fewer rows than 2 nt cost the same: the loads of the weights
+    return static_cast<double>(std::max<int64_t>(M, 2 * nt) * K) <= (group >= 128 ? limit : 1.5 * limit);
+  }
+  if (N > 16384) return N <= 32768 && group >= 128 && M * K <= 98304;
+  const double limit = 79872.0 + 65536.0 * (nt == 4 ? f2 : fill);
+  return static_cast<double>(M * K) <= (group >= 128 ? limit : 1.3 * limit);
+}
+
 int q4_rows_launch(const float* x, int64_t M, const int32_t* qw, const uint16_t* sc, float* y, const float* res,
                    int64_t N, int64_t K, int group, hipStream_t st) {
-  if (M <= 16) {
-    if (N <= 4096) return rows_go<1, 1>(x, M, qw, sc, y, res, N, K, group, st);
-    if (N <= 8192) return rows_go<1, 2>(x, M, qw, sc, y, res, N, K, group, st);
-    return rows_go<1, 4>(x, M, qw, sc, y, res, N, K, group, st);
-  }
-  if (N <= 4096) return rows_go<2, 1>(x, M, qw, sc, y, res, N, K, group, st);
-  if (N <= 8192) return rows_go<2, 2>(x, M, qw, sc, y, res, N, K, group, st);
-  return rows_go<2, 4>(x, M, qw, sc, y, res, N, K, group, st);
+  const auto go = M <= 16 ? (rows_nt(N) == 1 ? rows_go<1, 1> : rows_nt(N) == 2 ? rows_go<1, 2> : rows_go<1, 4>)
+                          : (rows_nt(N) == 1 ? rows_go<2, 1> : rows_nt(N) == 2 ? rows_go<2, 2> : rows_go<2, 4>);
+  return go(x, M, qw, sc, y, res, N, K, group, st);
 }
 
 }  // namespace q4

@@ -72,6 +72,19 @@ def test_linear_few_rows(dev, M, N, K, group):
         assert ((h.cpu().double() - ref).abs() <= bound).all(), (fn, M, N, K, group)
 
 
+@pytest.mark.parametrize("M,N,K,group", [(16, 520, 14336, 128), (2, 264, 28672, 64), (32, 64, 4096, 128), (12, 33000, 256, 32),
+                                         (20, 33000, 192, 64), (5, 8448, 16384, 128)])
+def test_linear_few_rows_on_tiles(dev, M, N, K, group):
+    """Few rows past the line of the one-launch kernel (long K, many columns), which run on the tiles when the
+    workspace holds their partials: every row and column of a tile that is mostly padding."""
+    x, qw, sc, res, ref, bound = linear_case(dev, M, N, K, group, M + N)
+    y = ops.q4_linear_ws(x, qw, sc, group, split=True)
+    assert ((y.cpu().double() - (ref - res.cpu().double())).abs() <= bound).all()
+    h = res.clone()
+    ops.q4_linear_ws(x, qw, sc, group, residual=h, out=h, split=True)
+    assert ((h.cpu().double() - ref).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("M,N,K,group", [(33, 40, 128, 32), (100, 515, 3072, 32), (257, 256, 256, 128), (300, 1030, 2048, 64),
                                          (385, 260, 4096, 256), (513, 3072, 1024, 128), (640, 5120, 192, 64),
                                          (1024, 4100, 512, 128), (19, 819, 6144, 128), (35, 1225, 3904, 64), (250, 3560, 128, 128),
