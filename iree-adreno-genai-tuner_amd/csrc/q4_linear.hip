@@ -1057,9 +1057,13 @@ double tile_time(int ti, int64_t wgs, int64_t steps, int group) {
   return us;
 }
 
-// The cheapest tile by tile_time, with a K split of up to 16 (pipelined tiles; whole groups, at least two
-// stages) whose partials fit `part_bytes`: their write and read cost 1.45 us per million, the launch that adds
-// them 2.0 us (none where the next kernel does it), and the estimate's error 5% in favour of no split.
+// The cheapest tile by tile_time, with a K split of up to 16, or 32 of at least nine stages (pipelined tiles;
+// whole groups, at least two stages), whose partials fit `part_bytes`: their write and read cost 1.45 us per
+// million, the launch that adds them 2.0 us (none where the next kernel does it), and the estimate's error 5% in
+// favour of no split (none up to 12 us, where the fit is high for few columns: 40x64x1024 unsplit 11.8, split
+// 10.4). Past 16 ranges their sum takes a second round of loads: 40x1024x4096 16.5 us in 16 ranges, 21.5 in 32 of
+// two stages; long ranges gain by the CUs that 16 leave idle, 20x1536x28672 g32 50.2 -> 38.2, 20x2048x18432 29.7 ->
+// 27.6.
 // Against the 64x64 and 32x64 tiles that ran all of these before (us, with the x split): 512x5120x3072
 // 78.8 -> 52.4, 512x16384x3072 197 -> 100 (group 32: 241 -> 135), 1024x5120x3072 127 -> 83, 1024x16384x3072
 // 375 -> 190. Against a split of every M <= 256 into about 256 workgroups of 64x256 (linear_split_plan), short
@@ -1072,14 +1076,17 @@ LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes,
   for (int ti = 0; ti < kNumLinWs; ++ti) {
     const LinWsTile& t = kLinWsTiles[ti];
     const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-    for (int64_t want = 1; want <= (t.pipe ? 16 : 1) && (want == 1 || tiles * (want - 1) < 256); ++want) {
+    for (int64_t want = 1; want <= (t.pipe ? 32 : 1) && (want == 1 || tiles * (want - 1) < 256); ++want) {
       int64_t nk_s = (nk + want - 1) / want;
       nk_s = (nk_s + gst - 1) / gst * gst;
       const int64_t S = (nk + nk_s - 1) / nk_s;
       const LinPlan p{ti, {static_cast<int>(S), S > 1 ? static_cast<int>(nk_s) : 0}};
-      if (S != want || (S > 1 && (nk_s < 2 || p.part_bytes(M, N) > part_bytes))) continue;
+      if (S != want || (S > 1 && (nk_s < (S > 16 ? 9 : 2) || p.part_bytes(M, N) > part_bytes))) continue;
       double us = tile_time(ti, tiles * S, nk_s, group);
-      if (S > 1) us = 1.05 * (us + (reduce ? 2.0 : 0.0) + 1.45e-6 * static_cast<double>(S * M * N));
+      if (S > 1) {
+        us += (reduce ? 2.0 : 0.0) + 1.45e-6 * static_cast<double>(S * M * N);
+        if (us > 12.0) us *= 1.05;
+      }
       if (us < best_us) best_us = us, best = p;
     }
   }

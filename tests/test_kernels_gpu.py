@@ -294,7 +294,7 @@ def test_q4_linear_ws_fp32_accuracy_every_tile(dev, M, N, K, group, kernel_overr
 
 @pytest.mark.parametrize("M,N,K,group", [(256, 5120, 3072, 128), (256, 3072, 3072, 128), (256, 3072, 8192, 128),
                                          (128, 5120, 3072, 128), (200, 3000, 3072, 128), (64, 256, 2048, 64),
-                                         (70, 1408, 1536, 32), (50, 520, 2048, 256), (256, 1000, 8192, 1024)])
+                                         (70, 1408, 1536, 32), (50, 520, 2048, 256), (256, 1000, 8192, 1024), (33, 521, 18432, 32)])
 def test_q4_linear_ws_k_split(dev, M, N, K, group):
     """With the larger workspace the prefill GEMM splits K over several workgroups per 64x256 tile and a
     second kernel adds the partials (fixed order) and the residual: same accuracy as the unsplit form,

@@ -486,10 +486,12 @@ def test_linear_ws_entries_cover_once(idx):
     (64, 256, 704, 64, 1), (33, 520, 1024, 256, 1), (256, 16384, 3072, 128, 1), (1024, 5120, 3072, 128, 1),  # no split
     (16, 1408, 256, 32, 1), (7, 3072, 3072, 128, 1), (24, 3072, 3072, 128, 1), (250, 3560, 128, 128, 1),  # one launch
     # few rows past the line of the one-launch kernel: long K, many columns; and next to it
-    (16, 4096, 14336, 128, 16), (4, 1536, 28672, 128, 16), (2, 8448, 14336, 128, 7), (24, 64, 4096, 128, 16),
+    (16, 4096, 14336, 128, 16), (4, 1536, 28672, 128, 32), (2, 8448, 14336, 128, 7), (24, 64, 4096, 128, 16),
     (32, 8448, 4096, 128, 7), (16, 4096, 8192, 128, 1), (8, 4096, 14336, 128, 1), (16, 4096, 12288, 32, 1), (32, 4096, 4096, 128, 1),
     (40, 96, 192, 96, 1),  # a group that is no power of two: the workspace-free kernel
-    (64, 256, 2048, 64, 16), (70, 1408, 1536, 32, 12), (50, 520, 2048, 256, 8), (256, 5120, 3072, 128, 3), (100, 515, 3072, 32, 16)])
+    (64, 256, 2048, 64, 16), (70, 1408, 1536, 32, 12), (50, 520, 2048, 256, 8), (256, 5120, 3072, 128, 3), (100, 515, 3072, 32, 16),
+    # more than 16 ranges only of nine stages or more; a split of little K for few columns
+    (20, 1536, 28672, 32, 32), (20, 2048, 18432, 128, 29), (40, 1024, 4096, 128, 16), (40, 64, 1024, 128, 8)])
 def test_linear_ws_split_bytes_is_what_the_call_writes(M, N, K, group, splits):
     """q4_linear_ws_split_bytes: the planes alone wherever the call adds no partials, else the planes (from a
     256-byte boundary) and `splits` times M N fp32 partials (whole float4s): nothing more is allocated per call."""
