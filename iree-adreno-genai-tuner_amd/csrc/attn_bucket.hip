@@ -935,13 +935,14 @@ __global__ __launch_bounds__(64 * kUnits, 2) void attn_prefill_mfma_kernel(
   };
 
   // Stage b's loads of this wave are complete when at most NST - 2 later stages' are in flight; the barrier
-  // publishes it and frees the buffer of stage b - 1, whose reads every wave has waited for. Stages past the
-  // last are issued too (out of range: no traffic), so the count is a constant.
+  // publishes it and frees the buffer of stage b - 1, whose reads every wave waits for here too (lgkmcnt(0)):
+  // that its MFMAs have used them by then is the compiler's present order, not a promise. Stages past the last
+  // are issued too (out of range: no traffic), so the count is a constant.
 #pragma unroll
   for (int b = 0; b < NST - 1; ++b) issue(b);
   for (int b = 0; b < nb; ++b) {
     constexpr int kWait = (NST - 2) * 2 * kLd;
-    __builtin_amdgcn_s_waitcnt((kWait & 15) | ((kWait >> 4) << 14) | (7 << 4) | (15 << 8));  // vmcnt only
+    __builtin_amdgcn_s_waitcnt((kWait & 15) | ((kWait >> 4) << 14) | (7 << 4));  // vmcnt(kWait), lgkmcnt(0)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");

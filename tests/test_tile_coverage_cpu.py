@@ -7,10 +7,15 @@ from the library (q4_gemv_config_info, q4_gemv_mx_config_info, gemm_f16_config_i
 q4_linear_ws_config_info); the index formulas restate the kernels (file:function cited per test).
 No GPU is needed."""
 
+import pathlib
+import re
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
-from q4llm._lib import config_table
+from q4llm._lib import LIB_PATH, config_table
 
 OOB = 0x80000000
 
@@ -514,6 +519,37 @@ def test_gemm_swizzle_is_bank_conflict_free(bk):
     # and the identity mapping (no swizzle) would not be: the check discriminates
     groups = {((r * row_b) // 16) % 16 for r in range(16)}
     assert len(groups) < 16
+
+
+# ------------------------------------------------------------------------------------------------
+# Prefill attention (csrc/attn_bucket.hip: attn_prefill_mfma_kernel)
+# ------------------------------------------------------------------------------------------------
+
+OBJDUMP = pathlib.Path("/opt/rocm/llvm/bin/llvm-objdump")
+
+
+@pytest.mark.skipif(not OBJDUMP.exists(), reason="needs llvm-objdump")
+def test_attn_ring_barrier_waits_for_lds_reads(tmp_path):
+    """The barrier that frees a buffer of the K/V ring (filled by direct loads) comes after a wait for this
+    wave's own LDS reads, whatever order the compiler gives the instructions that use them."""
+    so = tmp_path / "lib.so"
+    shutil.copy(LIB_PATH, so)
+    subprocess.run([OBJDUMP, "--offloading", so], check=True, capture_output=True)
+    found = 0
+    for code in sorted(tmp_path.glob("lib.so.*gfx950")):
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", code], check=True, capture_output=True, text=True).stdout
+        name, before = "", ""
+        for line in text.splitlines():
+            head = re.match(r"[0-9a-f]+ <(.*)>:", line)
+            ins = line.split("//")[0].strip()
+            if head:
+                name = head[1]
+            elif "attn_prefill_mfma_kernel" in name and ins:
+                if ins.startswith("s_barrier"):
+                    assert before.startswith("s_waitcnt") and "vmcnt" in before and "lgkmcnt(0)" in before, (name, before)
+                    found += 1
+                before = ins
+    assert found == 2  # one per head size
 
 
 # ------------------------------------------------------------------------------------------------
