@@ -401,6 +401,11 @@ int gemm_f16_nt_cfg(const uint16_t* A, const uint16_t* B, uint16_t* C, int64_t M
  *                           per 16-row block, grid-stride (q4_gemv_mx_num_configs entries)
  *   gemm_f16_config_info:   BM, BN, wave rows, wave columns, stages, BK, pipelined substeps
  *   q4_linear_ws_config_info: BM, BN, wave rows, wave columns, stages, k-split, pipelined (0/1) */
+/* How the projections of one step of C tokens and bucket L run on those tiles: plan[2 i] = q4_linear_ws tile
+ * entry and plan[2 i + 1] = K ranges of qkv, o, gate/up and down (i = 0 .. 3). More than one range: the
+ * next kernel adds their partials; 0 ranges: gate/up with SwiGLU as its epilogue; -1, -1: not on the tiles
+ * (decode, a few rows, sizes that they do not take). */
+int q4llm_step_plan(const q4llm_model* m, int C, int L, int* plan);
 int q4_gemv_config_info(int cfg, int* info);
 int q4_gemv_mx_num_configs(void);
 int q4_gemv_mx_config_info(int cfg, int* info);

@@ -80,6 +80,9 @@ size_t linear_split_part_bytes(int64_t M, int64_t N, int64_t K, int group);
 // that q4_linear_ws writes on its fastest plan for this shape (0: no split)
 size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group);
 
+// Tile entry and K ranges (0: the SwiGLU epilogue) of a model step's projection with part_bytes of partials.
+void linear_step_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool swiglu, int* tile, int* ranges);
+
 // q4_linear_ws's GEMM on given planes (power-of-two group); with `part` (part_bytes, 16-byte aligned) it
 // may split K and reduce the partials in a second kernel.
 // With `deferred` not null, a K split leaves its partials in `part` unreduced and sets *deferred to the

@@ -1093,9 +1093,20 @@ LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes,
   return best;
 }
 
-}  // namespace
+// The plan that runs: tile_plan's, or the tile of the Q4_DBG_LINEAR_TILE override (no K split).
+LinPlan running_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool reduce) {
+  const int ov = debug_override(Q4_DBG_LINEAR_TILE);
+  if (ov >= 0 && ov < kNumLinWs) return LinPlan{ov, {1, 0}};
+  return tile_plan(M, N, K, group, std::min<size_t>(part_bytes, size_t{1} << 33), reduce);
+}
 
-namespace {
+// Chunks whose gate/up projection takes the SwiGLU epilogue: its tile alone gives one workgroup per CU.
+bool swiglu_epilogue(int64_t M, int64_t N) {
+  constexpr LinWsTile t = kLinWsTiles[kSplitTile];
+  if (debug_set(Q4_DBG_LINEAR_TILE) || debug_flag(Q4_DBG_SWIGLU_UNFUSED)) return false;
+  return M <= 256 && ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) >= 256 && N % t.bn == 0 && (N / 2) % 32 == 0;
+}
+
 // Calls of q4_linear_ws that one launch without planes or partials serves better: a few rows (q4_rows_wins;
 // short of the partials that the tiles need, all that the kernel takes), and K of at most two stages while its 64x64 tiles run at once, where the launch that splits x costs more than it
 // gives: 250x3560x128 7.8 -> 6.2 us, 33x256x128 6.4 -> 5.5 (two rounds of tiles, 700x3560x128: 12.7 | 14.9);
@@ -1112,6 +1123,13 @@ size_t linear_plan_part_bytes(int64_t M, int64_t N, int64_t K, int group) {
   return one_launch(M, N, K, group, SIZE_MAX) ? 0 : tile_plan(M, N, K, group, SIZE_MAX, true).part_bytes(M, N);
 }
 
+void linear_step_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes, bool swiglu, int* tile, int* ranges) {
+  const bool epi = swiglu && swiglu_epilogue(M, N);
+  const LinPlan p = epi ? LinPlan{kSplitTile, {0, 0}} : running_plan(M, N, K, group, (M * N) % 4 ? 0 : part_bytes, false);
+  *tile = p.tile;
+  *ranges = p.split.n_split;
+}
+
 // The pipelined GEMM on x given as fp16 (hi, lo) planes (store_x_planes layout, [M, K] each);
 // power-of-two groups only. tile_plan picks the tile and, with a partial buffer `part` that holds it,
 // the K split, whose partials linear_reduce_kernel adds. Q4_DBG_LINEAR_TILE overrides (no K split). `t16`
@@ -1125,9 +1143,7 @@ int q4_linear_planes(const uint16_t* xh, const uint16_t* xl, int64_t M, const in
   // what the partials and linear_reduce_kernel (a caller's next kernel: whole float4s too) need
   const bool can_split = part && (!deferred || (M * N) % 4 == 0) && aligned(part, 16) && aligned(y, 16) &&
                          (!res || aligned(res, 16));
-  LinPlan plan = tile_plan(M, N, K, group, can_split ? std::min<size_t>(part_bytes, size_t{1} << 33) : 0, !t16);
-  const int ov = debug_override(Q4_DBG_LINEAR_TILE);
-  if (ov >= 0 && ov < kNumLinWs) plan = LinPlan{ov, {1, 0}};
+  const LinPlan plan = running_plan(M, N, K, group, can_split ? part_bytes : 0, !t16);
   const int ti = plan.tile, S = plan.split.n_split;
   const LinWsTile& t = kLinWsTiles[ti];
   const int tiles_n = static_cast<int>((N + t.bn - 1) / t.bn);
@@ -1162,10 +1178,8 @@ int q4_linear_planes_swiglu(const uint16_t* xh, const uint16_t* xl, int64_t M, c
                             const T16Src* t16) {
   if (int e = planes_args(xh, xl, M, qw, sc, N, K, group)) return e;
   if (!oh || !ol) return Q4_ERR_NULL;
-  if (debug_set(Q4_DBG_LINEAR_TILE) || debug_flag(Q4_DBG_SWIGLU_UNFUSED)) return Q4_ERR_UNSUPPORTED;
+  if (!swiglu_epilogue(M, N) || ol != oh + M * (N / 2)) return Q4_ERR_UNSUPPORTED;
   constexpr LinWsTile t = kLinWsTiles[kSplitTile];
-  const int64_t wide = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-  if (!(M <= 256 && wide >= 256) || N % t.bn || (N / 2) % 32 || ol != oh + M * (N / 2)) return Q4_ERR_UNSUPPORTED;
   const bool use_t16 = t16_usable(t16, N, group, Q4_PAIR_SWIGLU);
   const LinWsFn fn = use_t16 ? lin_ws_t16_fn<1, kSplitTile>() : q4_linear_ws_kernel<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks, 1, t.pipe>;
   constexpr size_t lds = LinWsCfg<t.bm, t.bn, t.wm, t.wn, t.nst, t.ks>::kLds;

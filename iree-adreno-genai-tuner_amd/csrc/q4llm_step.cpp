@@ -101,6 +101,20 @@ bool scales_on_words(const q4llm_model* m) {
   return true;
 }
 
+// Whether a chunk's projections read fp16 (hi, lo) planes written by the kernels before them. A few rows take
+// the other path, whose projections are one launch each and read fp32 rows: what the tiled path fills with
+// padding and K splits costs more there. Measured (6 layers of dim 3072, inter 8192, group 128 | 4 layers of dim
+// 1024, inter 3072, group 32; tiled -> this, us): C = 2 527 -> 410 | 315 -> 183, C = 8 542 -> 462 | 325 -> 203,
+// C = 16 566 -> 533 | 337 -> 219. From 17 rows on while C dim <= 65536 (inter 4096: C = 17 535 -> 509, C = 24
+// 560 -> 558, C = 32 592 -> 605; dim 1024: C = 32 365 -> 262).
+bool prefill_planes(const q4llm_model* m, int C) {
+  const int D = m->dim, nq_w = m->n_heads * m->head_dim;
+  const bool few_rows = q4::q4_rows_takes(C, std::max(D, std::max(nq_w, m->inter))) &&
+                        (C <= 16 || static_cast<int64_t>(C) * D <= 65536);
+  return C > 1 && !few_rows && (m->group & (m->group - 1)) == 0 && linear_fits(D, m->group) &&
+         linear_fits(nq_w, m->group) && linear_fits(m->inter, m->group) && scales_on_words(m);
+}
+
 int check_model(const q4llm_model* m) {
   if (!m || !m->layers || !m->embed_q || !m->embed_s || !m->ln_f || !m->cos_t || !m->sin_t) return Q4_ERR_NULL;
   if (m->dim <= 0 || m->n_layers <= 0 || m->n_heads <= 0 || m->n_kv <= 0 || m->head_dim <= 0 || m->inter <= 0 ||
@@ -151,6 +165,23 @@ extern "C" int q4llm_step_workspace_bytes(const q4llm_model* m, int C, int L, si
   return Q4_OK;
 }
 
+extern "C" int q4llm_step_plan(const q4llm_model* m, int C, int L, int* plan) {
+  if (!plan) return Q4_ERR_NULL;
+  size_t bytes = 0;
+  if (int st = q4llm_step_workspace_bytes(m, C, L, &bytes)) return st;
+  Layout lo;
+  if (int st = layout_for(m, C, L, &lo)) return st;
+  const int64_t nq = m->n_heads * m->head_dim, qkv = nq + 2 * m->n_kv * m->head_dim;
+  const int64_t shapes[4][2] = {{qkv, m->dim}, {m->dim, nq}, {2 * static_cast<int64_t>(m->inter), m->dim}, {m->dim, m->inter}};
+  const bool planes = prefill_planes(m, C);
+  for (int i = 0; i < 4; ++i) {
+    plan[2 * i] = plan[2 * i + 1] = -1;
+    if (planes)
+      q4::linear_step_plan(C, shapes[i][0], shapes[i][1], m->group, lo.part_bytes, i == 2, &plan[2 * i], &plan[2 * i + 1]);
+  }
+  return Q4_OK;
+}
+
 namespace {
 // One step; with `advance` not null, start[0] += C on the device after the next token is written
 // (q4llm_step_feed).
@@ -197,14 +228,7 @@ int step_impl(const q4llm_model* m, const int32_t* tokens, int C, const int32_t*
   // Prefill with a power-of-two group: the norms, the attention merge and SwiGLU write their results
   // straight as the fp16 (hi, lo) planes the following projection reads (in the lin workspace).
   const int kmax = std::max(D, std::max(nq_w, m->inter));
-  // A few rows take the other path, whose projections are one launch each and read fp32 rows: what the tiled
-  // path fills with padding and K splits costs more there. Measured (6 layers of dim 3072, inter 8192, group
-  // 128 | 4 layers of dim 1024, inter 3072, group 32; tiled -> this, us): C = 2 527 -> 410 | 315 -> 183, C = 8
-  // 542 -> 462 | 325 -> 203, C = 16 566 -> 533 | 337 -> 219. From 17 rows on while C dim <= 65536 (inter 4096:
-  // C = 17 535 -> 509, C = 24 560 -> 558, C = 32 592 -> 605; dim 1024: C = 32 365 -> 262).
-  const bool few_rows = q4::q4_rows_takes(C, kmax) && (C <= 16 || static_cast<int64_t>(C) * D <= 65536);
-  const bool planes = C > 1 && !few_rows && (m->group & (m->group - 1)) == 0 && linear_fits(D, m->group) &&
-                      linear_fits(nq_w, m->group) && linear_fits(m->inter, m->group) && scales_on_words(m);
+  const bool planes = prefill_planes(m, C);
   uint16_t* xh = static_cast<uint16_t*>(lin_ws);
   uint16_t* xl = xh + static_cast<size_t>(C) * kmax;
   const hipStream_t st = static_cast<hipStream_t>(stream);

@@ -65,6 +65,7 @@ SIGNATURES = {
     "argmax_workspace_bytes": [i64, C.POINTER(sz)],
     "argmax_f32": [p, i64, p, p, sz, p],
     "q4llm_step_workspace_bytes": [p, i32, i32, C.POINTER(sz)],
+    "q4llm_step_plan": [p, i32, i32, p],
     "q4llm_step": [p, p, i32, p, p, p, i32, p, p, p, sz, p],
     "q4llm_advance_position": [p, i32, p],
     "q4llm_step_feed": [p, p, i32, p, p, p, i32, p, p, p, sz, p],

@@ -338,6 +338,13 @@ class LlamaQ4(nn.Module):
             self._ws[key] = torch.empty(b.value, dtype=torch.uint8, device=self.device)
         return self._ws[key]
 
+    def step_plan(self, Cn, L):
+        """((tile entry, K ranges) of the qkv, o, gate/up and down projections) of a step of Cn tokens, as
+        q4llm_step_plan gives them."""
+        plan = (C.c_int * 8)()
+        LIB.call("q4llm_step_plan", C.byref(self.descriptor()), Cn, L, plan)
+        return tuple((plan[2 * i], plan[2 * i + 1]) for i in range(4))
+
     def _cache_ptrs(self, caches):
         if len(caches) != 2 * self.n_layers:
             raise ValueError(f"expected {2 * self.n_layers} cache tensors, got {len(caches)}")

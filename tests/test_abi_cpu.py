@@ -83,6 +83,12 @@ def test_step_validation_without_device():
     assert f("q4llm_step_workspace_bytes")(C.byref(m), 16, 256, C.byref(b)) == ERR["RANGE"]  # L > max_ctx
     caches = (C.c_void_p * 2)(FAKE, FAKE)
     assert f("q4llm_step")(C.byref(m), FAKE, 16, FAKE, FAKE, caches, 64, FAKE, None, FAKE, 16, None) == ERR["WORKSPACE"]
+    plan = (C.c_int * 8)()
+    assert f("q4llm_step_plan")(C.byref(m), 100, 128, plan) == 0 and list(plan) != [-1] * 8
+    for few in (1, 16):  # decode and a few rows: not on the tiles
+        assert f("q4llm_step_plan")(C.byref(m), few, 128, plan) == 0 and list(plan) == [-1] * 8
+    assert f("q4llm_step_plan")(C.byref(m), 100, 256, plan) == ERR["RANGE"]
+    assert f("q4llm_step_plan")(C.byref(m), 100, 128, None) == ERR["NULL"]
     bad = (_LayerC * 1)(_LayerC(*([FAKE] * 9 + [0])))
     m2 = _ModelC(256, 1, 4, 2, 64, 704, 1024, 32, 128, 1e-5, FAKE, FAKE, FAKE, FAKE, FAKE, C.cast(bad, C.c_void_p))
     assert f("q4llm_step_workspace_bytes")(C.byref(m2), 16, 64, C.byref(b)) == ERR["NULL"]

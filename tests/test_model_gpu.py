@@ -18,12 +18,26 @@ pytestmark = pytest.mark.gpu
 GOLD = pathlib.Path(__file__).parent / "golden"
 
 
-def build_pair(cfg, group, max_ctx, seed=0, std=0.2):
+def build_pair(cfg, group, max_ctx, seed=0, std=None):
+    """Weights of std 0.2; past hidden size 1024 such that a projection's gain, std sqrt(hidden), stays that of
+    1024 (6.4). Scores are q . k / sqrt(hd) of entries of that size: std gain^2 = 41, where one fp16 ulp
+    (2^-11) of the differently rounded K entries moves a score by up to gain^2 2^-11 = 0.02 and the logits by
+    less than their tolerance; at 0.2 and hidden 3072 (gain 11) the same flips move scores by 0.06."""
+    std = std or min(0.2, 6.4 / cfg["hidden_size"] ** 0.5)
     sd = synth.SyntheticWeights(cfg, seed, std=std)
     dense = {k: sd[k] for k in sd.keys()}
     ours = LlamaQ4(None, group=group, max_ctx=max_ctx, sd=dense, cfg=cfg)
     ref = R.LlamaQ4Ref(cfg, dense, group=group, max_ctx=max_ctx, rope=(ours.cos.cpu(), ours.sin.cpu()))
     return ours, ref
+
+
+# K-split projections (their ranges at 128 and 256 rows: test_prefill_deferred_partials_...)
+SPLIT_DIMS = dict(hidden_size=2048, intermediate_size=4096, num_attention_heads=16, num_key_value_heads=8, head_dim=128)
+
+
+def ranges(model, chunk, L):
+    """K ranges of the qkv, o, gate/up and down projections of a chunk (0: gate/up with the SwiGLU epilogue)."""
+    return [r for _, r in model.step_plan(chunk, L)]
 
 
 def tol(ref):
@@ -164,6 +178,7 @@ def test_prefill_swiglu_epilogue_matches_two_kernels_and_oracle(dev, kernel_over
     (the swiglu_unfused override), and the oracle's next token with logits within the per-op tolerance."""
     cfg = dict(synth.TINY, intermediate_size=8192, num_hidden_layers=2)
     ours, ref = build_pair(cfg, 32, 256)
+    assert ranges(ours, 256, 256)[2] == 0
     prompt = synth.prompt_ids(256, cfg["vocab_size"], seed=3)
     toks = torch.tensor([prompt], dtype=torch.int32)
     start, last = torch.tensor([0], dtype=torch.int32), torch.tensor([255], dtype=torch.int32)
@@ -184,11 +199,12 @@ def test_prefill_swiglu_epilogue_matches_two_kernels_and_oracle(dev, kernel_over
 def test_prefill_chunk128_k_split_paths_vs_oracle(dev, kernel_override):
     """A 128-row chunk takes every K-split path of the prefill step: qkv, o and down split and completed
     by the RoPE / rms_norm kernels after them, and gate/up (too few 64x256 tiles at 128 rows for its
-    SwiGLU epilogue) split 2 ways, its partials added by the silu_mul kernel: bit-identical to adding
+    SwiGLU epilogue) split too, its partials added by the silu_mul kernel: bit-identical to adding
     them with the reduce kernel first (the swiglu_unfused override). Two chunks (the second reading the first's
     caches), next token and logits against the oracle."""
-    cfg = dict(synth.TINY, intermediate_size=8192, num_hidden_layers=2)
+    cfg = dict(synth.TINY, num_hidden_layers=2, **SPLIT_DIMS)
     ours, ref = build_pair(cfg, 32, 256)
+    assert min(ranges(ours, 128, 256)) > 1
     prompt = synth.prompt_ids(256, cfg["vocab_size"], seed=5)
     c_ours, c_two, c_ref = ours.new_caches(), ours.new_caches(), ref.new_caches()
     for s0 in (0, 128):
@@ -225,20 +241,25 @@ def test_prefill_few_rows_vs_oracle(dev, cfg_kw, chunk):
         assert (l_o.cpu() - r_l).abs().max().item() <= tol(r_l), s0
 
 
-@pytest.mark.parametrize("cfg_kw,chunk", [
-    # qkv and o: 4 partials each; down: 128 (past the 12 loaded with the row: the tail loop); gate/up: 2
-    (dict(intermediate_size=8192), 128),
-    # qkv 8 (RoPE kernel), o 4 and down 7 (rms_norm, 6-wide and 12-wide batches), gate/up 8 (silu_mul)
-    (dict(hidden_size=512, intermediate_size=448), 128),
-    (dict(hidden_size=512, intermediate_size=448), 256),
+@pytest.mark.parametrize("cfg_kw,chunk,splits", [
+    # K ranges of qkv, o, gate/up and down. rms_norm (o, down) loads up to 6 or 12 partials with the row and the
+    # rest in a loop; RoPE (qkv) and silu_mul (gate/up) 8, then a loop
+    (SPLIT_DIMS, 128, [8, 11, 4, 16]),
+    (SPLIT_DIMS, 256, [4, 8, 2, 8]),
+    (SPLIT_DIMS, 64, [11, 16, 8, 16]),
+    (dict(SPLIT_DIMS, hidden_size=3072, intermediate_size=2048), 256, [4, 5, 4, 5]),
+    (dict(SPLIT_DIMS, hidden_size=3072, intermediate_size=2048), 64, [12, 11, 12, 11]),
+    # only down splits
+    (dict(intermediate_size=8192), 128, [1, 1, 1, 16]),
 ])
-def test_prefill_deferred_partials_bit_identical_to_reduce_kernel(dev, kernel_override, cfg_kw, chunk):
+def test_prefill_deferred_partials_bit_identical_to_reduce_kernel(dev, kernel_override, cfg_kw, chunk, splits):
     """The kernels that add a K-split projection's partials themselves (RoPE + KV write after qkv,
     rms_norm after o and down, silu_mul after a split gate/up, the final norm's selected row) give the
     same bits as reducing each projection with linear_reduce_kernel first and running the plain
     kernels (the reduce_splits override): logits, next token and every K/V cache, chunk after chunk."""
     cfg = dict(synth.TINY, num_hidden_layers=2, **cfg_kw)
     ours, ref = build_pair(cfg, 32, 256)
+    assert ranges(ours, chunk, 256) == splits
     prompt = synth.prompt_ids(256, cfg["vocab_size"], seed=7)
     c_def, c_red, c_ref = ours.new_caches(), ours.new_caches(), ref.new_caches()
     for s0 in range(0, 256, chunk):
@@ -256,29 +277,46 @@ def test_prefill_deferred_partials_bit_identical_to_reduce_kernel(dev, kernel_ov
         assert (l_d.cpu() - r_l).abs().max().item() <= tol(r_l), s0
 
 
-@pytest.mark.parametrize("chunk", [256, 128])
-def test_prefill_t16_source_matches_reference_layout(dev, kernel_override, chunk):
-    """Prefill projections on the 64x256 tile read the decode T16 copies (RoPE-paired qkv, plain o and
-    down, SwiGLU-paired gate/up) instead of the reference layout: the same sums in the same order, so
-    the logits and the K/V caches are bit-identical to the prefill_ref_layout override (256-row chunk: the SwiGLU
-    epilogue; 128 rows: every projection K-split), and the token matches the oracle."""
-    cfg = dict(synth.TINY, hidden_size=1024, num_attention_heads=8, num_key_value_heads=4, head_dim=128,
-               intermediate_size=8192, num_hidden_layers=2)
-    ours, ref = build_pair(cfg, 128, 256)
-    assert all((i, nm) in ours.t16 for i in range(2) for nm in ("wqkv", "wo", "wgu", "wdown"))
-    prompt = synth.prompt_ids(256, cfg["vocab_size"], seed=11)
+T16_DIMS = dict(hidden_size=1024, num_attention_heads=8, num_key_value_heads=4, head_dim=128, intermediate_size=8192)
+
+
+@pytest.mark.parametrize("cfg_kw,group,chunk,tile,plan", [
+    # (tile entry, K ranges) of qkv, o, gate/up and down; entries 0 (128x256) and 2 (64x256) read T16
+    (T16_DIMS, 128, 256, None, ((1, 1), (1, 1), (2, 0), (2, 16))),  # gate/up: the SwiGLU epilogue
+    (T16_DIMS, 128, 128, None, ((1, 1), (2, 8), (2, 1), (2, 16))),
+    (dict(T16_DIMS, intermediate_size=1024), 128, 100, None, ((2, 8),) * 4),  # every projection K-split
+    (T16_DIMS, 128, 300, None, ((1, 1), (1, 1), (0, 1), (1, 1))),  # more than 256 rows: gate/up on 128x256
+    (dict(hidden_size=256, num_attention_heads=64, num_key_value_heads=32, head_dim=128, intermediate_size=4096), 32, 300,
+     None, ((0, 1), (1, 1), (1, 1), (1, 1))),  # qkv (RoPE pairing) on 128x256
+    # every projection on one of the two tiles
+    (T16_DIMS, 128, 300, 0, ((0, 1),) * 4),
+    (T16_DIMS, 128, 100, 2, ((2, 1),) * 4),
+    (dict(T16_DIMS, intermediate_size=1024), 128, 130, 0, ((0, 1),) * 4),
+])
+def test_prefill_t16_source_matches_reference_layout(dev, kernel_override, cfg_kw, group, chunk, tile, plan):
+    """Prefill projections on the 64x256 and 128x256 tiles read the decode T16 copies (RoPE-paired qkv, plain o
+    and down, SwiGLU-paired gate/up) instead of the reference layout: the same sums in the same order, so
+    the logits and the K/V caches are bit-identical to the prefill_ref_layout override, and the token matches
+    the oracle."""
+    cfg = dict(synth.TINY, num_hidden_layers=2, **cfg_kw)
+    ours, ref = build_pair(cfg, group, 512)
+    kernel_override("linear_tile", tile)
+    L = 256 if chunk <= 256 else 512
+    assert ours.step_plan(chunk, L) == plan
+    assert all((i, nm) in ours.t16 for i in range(2) for nm, (t, _) in zip(("wqkv", "wo", "wgu", "wdown"), plan) if t != 1)
+    prompt = synth.prompt_ids(512, cfg["vocab_size"], seed=11)
     toks = torch.tensor([prompt[:chunk]], dtype=torch.int32)
     start, last = torch.tensor([0], dtype=torch.int32), torch.tensor([chunk - 1], dtype=torch.int32)
     c_t = ours.new_caches()
-    n_t, l_t = ours.step(toks, start, last, c_t, 256)
+    n_t, l_t = ours.step(toks, start, last, c_t, L)
     kernel_override("prefill_ref_layout", 1)
     c_r = ours.new_caches()
-    n_r, l_r = ours.step(toks, start, last, c_r, 256)
+    n_r, l_r = ours.step(toks, start, last, c_r, L)
     kernel_override("prefill_ref_layout", None)
     assert torch.equal(l_t, l_r) and int(n_t.item()) == int(n_r.item())
     for a, b in zip(c_t, c_r):
         assert torch.equal(a, b)
-    r_n, r_l = ref.step(toks, start, last, ref.new_caches(), 256)
+    r_n, r_l = ref.step(toks, start, last, ref.new_caches(), L)
     assert int(n_t.item()) == int(r_n.item())
     assert (l_t.cpu() - r_l).abs().max().item() <= tol(r_l)
 

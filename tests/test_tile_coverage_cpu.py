@@ -385,21 +385,41 @@ def test_tile_entries_keep_their_index():
     assert [lin[i] for i in (1, 2)] == [(32, 64, 1, 2, 4, 2, 0), (64, 256, 2, 4, 4, 1, 1)]
 
 
+def lib_gemm_splits(M, N, K):
+    """K ranges that the library's rule takes for this problem, from the workspace it asks for."""
+    from q4llm import ops
+    need = ops.gemm_f16_nt_ws_bytes(M, N, K)
+    assert need % (4 * M * N) == 0
+    return max(need // (4 * M * N), 1)
+
+
+SPLIT_SIZES = [(256, 5120, 3072), (256, 3072, 8192), (256, 16384, 3072), (1024, 5120, 3072), (1024, 1024, 1024), (128, 3072, 3072),
+               (4096, 64, 1024), (16, 4096, 4096), (256, 256, 8192), (768, 768, 768), (250, 3074, 8192), (300, 520, 776)]
+
+
+@pytest.mark.parametrize("idx", range(len(config_table("gemm"))))
+def test_gemm_split_of_an_entry_matches_the_library(idx, kernel_override):
+    """The split by size that the replays above restate is the library's, on every tile entry."""
+    kernel_override("gemm_tile", idx)
+    for M, N, K in SPLIT_SIZES:
+        assert lib_gemm_splits(M, N, K) == gemm_split(config_table("gemm")[idx], M, N, K)[0], (M, N, K)
+
+
 def test_gemm_split_rule_fills_the_cus():
-    """The automatic K split of the 256-row config-3 shapes on the pipelined 128x128 entry."""
-    cfg = next(c for c in config_table("gemm") if c[:6] == (128, 128, 2, 2, 4, 64) and c[6])
-    assert gemm_split(cfg, 256, 5120, 3072) == (3, 16)   # 80 tiles x 3
-    assert gemm_split(cfg, 256, 3072, 8192) == (5, 26)   # 48 tiles x 5 (last range 24 steps)
-    assert gemm_split(cfg, 256, 16384, 3072) == (1, 0)   # 256 tiles fill the CUs
-    assert gemm_split(cfg, 1024, 5120, 3072) == (1, 0)   # no split from 512 rows on
+    """The library's own rule: K ranges of the config-3 shapes and of sizes around its lines."""
+    assert lib_gemm_splits(256, 5120, 3072) == 3
+    assert lib_gemm_splits(256, 3072, 8192) == 5
+    assert lib_gemm_splits(512, 3072, 8192) == 5   # past 512 rows too where the tiles leave CUs idle
+    for full in ((256, 16384, 3072), (1024, 5120, 3072), (2048, 3072, 8192), (4096, 4096, 4096)):
+        assert lib_gemm_splits(*full) == 1, full   # the tiles fill the CUs
+    assert lib_gemm_splits(250, 3074, 8192) == 1   # N % 4: the launch that adds the partials takes four columns
     # problems under 4 GFLOP (the reference's S1-S8) take the 64x64 entry and about 256 workgroups
-    c64 = next(c for c in config_table("gemm") if c[:2] == (64, 64))
-    assert gemm_split(c64, 1024, 1024, 1024) == (1, 0)   # S1: 256 tiles
-    assert gemm_split(c64, 128, 3072, 3072) == (3, 16)   # S2: 96 tiles x 3
-    assert gemm_split(c64, 4096, 64, 1024) == (2, 8)     # S3: 64 tiles x 2 (8-step ranges)
-    assert gemm_split(c64, 16, 4096, 4096) == (4, 16)    # S4: 64 tiles x 4
-    assert gemm_split(c64, 256, 256, 8192) == (16, 8)    # S5: 16 tiles x 16
-    assert gemm_split(c64, 768, 768, 768) == (1, 0)      # S8: 144 tiles, 12 steps
+    assert lib_gemm_splits(1024, 1024, 1024) == 1  # S1: 256 tiles
+    assert lib_gemm_splits(128, 3072, 3072) == 3   # S2: 96 tiles x 3
+    assert lib_gemm_splits(4096, 64, 1024) == 2    # S3: 64 tiles x 2 (8-step ranges)
+    assert lib_gemm_splits(16, 4096, 4096) == 4    # S4: 64 tiles x 4
+    assert lib_gemm_splits(256, 256, 8192) == 16   # S5: 16 tiles x 16
+    assert lib_gemm_splits(768, 768, 768) == 1     # S8: 144 tiles, 12 steps
 
 
 # ------------------------------------------------------------------------------------------------
@@ -597,16 +617,24 @@ def t16_pack(qbytes, sc, N, K, group, pairing, hd):
     return tiles.reshape(-1), scales.reshape(-1), n_t16, n_tiles, nseg
 
 
+T16_ENTRIES = [i for i, cfg in enumerate(config_table("linear_ws")) if cfg[6]]  # the pipelined tiles
+
+
+def test_t16_entries():
+    assert {config_table("linear_ws")[i][:2] for i in T16_ENTRIES} == {(64, 256), (128, 256)}
+
+
+@pytest.mark.parametrize("entry", T16_ENTRIES)
 @pytest.mark.parametrize("pairing,N,K,group", [(0, 200, 1024, 128), (2, 256 + 64, 768, 128), (1, 512 + 32, 512, 32),
                                                (0, 96, 1536, 32)])
-def test_linear_ws_t16_loads_and_outputs(pairing, N, K, group):
+def test_linear_ws_t16_loads_and_outputs(pairing, N, K, group, entry):
     """Every 1 KB weight load of a 64-k stage of 32 virtual columns brings, for LDS row r (lane / 2), the
     64 nibbles of weight row t16_row(column) at that stage; every scale slot holds the fp16 scale of that
     row and the stage's group; and the epilogue writes each virtual column to t16_row (EPI 0, every
-    pairing) and, for the SwiGLU epilogue, each pair once from the lane holding gate with up 8 columns
+    pairing) and, for the SwiGLU epilogue (64x256), each pair once from the lane holding gate with up 8 columns
     away."""
     hd = 64
-    cfg = config_table("linear_ws")[-1]
+    cfg = config_table("linear_ws")[entry]
     bm, bn, wm, wn, nst, ks_n, pipe = cfg
     assert bn % 128 == 0 and ks_n == 1 and pipe == 1
     waves = wm * wn
