@@ -1041,15 +1041,21 @@ struct LinPlan {
 // Estimated time (us) of `wgs` workgroups of `steps` 64-k stages each on tile entry `ti`: rounds of at most
 // `cap` workgroups, each stage's time growing with how many of them run (the matrix cores' clock and the
 // L2 are shared). Fitted (relative error 3% in the median, 10% at the 90th percentile) to 400 shapes of M
-// 33-1024, N 256-16384, K 128-8192 at groups 128 and 32, splits of 1-16, graph replays over rotated weights.
+// 33-1024, N 256-16384, K 128-8192 at groups 128 and 32, splits of 1-16, graph replays over rotated weights. The
+// other groups' steps differ from those by what the tiles' times at K 2048, 4096 and 8192 do (64x256, 128
+// workgroups: 1.27 us a step at group 32, 1.06 at 64, 0.83 at 128, 0.95 at 256). With the rates of 32 for 64 and
+// of 128 for 256, 87x13092x5568 group 64 took 88 us, now 60, and 131x3131x2048 group 256 22.2, now 19.5.
 double tile_time(int ti, int64_t wgs, int64_t steps, int group) {
   struct Rate {
     double fixed, round, step, load;
     int cap;
   };
-  constexpr Rate kRates[2][3] = {{{8.7, 0, 1.318, 0.200, 256}, {5.7, 1.0, 0.352, 0.112, 768}, {7.2, 0, 0.801, 0.201, 256}},
-                                 {{8.7, 0, 2.030, 0.100, 256}, {5.7, 1.0, 0.397, 0.125, 768}, {7.3, 0, 1.258, 0.167, 256}}};
-  const Rate& r = kRates[group >= 128 ? 0 : 1][ti];
+  // groups of 32, 64, 128, more: how often sums are scaled, and (128 alone) without zeroing or branches
+  constexpr Rate kRates[4][3] = {{{8.7, 0, 2.030, 0.100, 256}, {5.7, 1.0, 0.397, 0.125, 768}, {7.3, 0, 1.258, 0.167, 256}},
+                                 {{8.7, 0, 1.730, 0.100, 256}, {5.7, 1.0, 0.397, 0.125, 768}, {7.3, 0, 1.050, 0.167, 256}},
+                                 {{8.7, 0, 1.318, 0.200, 256}, {5.7, 1.0, 0.352, 0.112, 768}, {7.2, 0, 0.801, 0.201, 256}},
+                                 {{8.7, 0, 1.370, 0.200, 256}, {5.7, 1.0, 0.352, 0.112, 768}, {7.2, 0, 0.880, 0.201, 256}}};
+  const Rate& r = kRates[group <= 32 ? 0 : group <= 64 ? 1 : group <= 128 ? 2 : 3][ti];
   const int64_t full = wgs / r.cap, rest = wgs % r.cap;
   double us = r.fixed + static_cast<double>(full - (rest ? 0 : 1)) * r.round;
   us += static_cast<double>(full * steps) * (r.step + r.load * r.cap / 256.0);
@@ -1057,7 +1063,7 @@ double tile_time(int ti, int64_t wgs, int64_t steps, int group) {
   return us;
 }
 
-// The cheapest tile by tile_time, with a K split of up to 16, or 32 of at least nine stages (pipelined tiles;
+// The cheapest tile by tile_time, with a K split of up to 16, or 32 of at least eight stages (pipelined tiles;
 // whole groups, at least two stages), whose partials fit `part_bytes`: their write and read cost 1.45 us per
 // million, the launch that adds them 2.0 us (none where the next kernel does it), and the estimate's error 5% in
 // favour of no split (none up to 12 us, where the fit is high for few columns: 40x64x1024 unsplit 11.8, split
@@ -1081,7 +1087,7 @@ LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes,
       nk_s = (nk_s + gst - 1) / gst * gst;
       const int64_t S = (nk + nk_s - 1) / nk_s;
       const LinPlan p{ti, {static_cast<int>(S), S > 1 ? static_cast<int>(nk_s) : 0}};
-      if (S != want || (S > 1 && (nk_s < (S > 16 ? 9 : 2) || p.part_bytes(M, N) > part_bytes))) continue;
+      if (S != want || (S > 1 && (nk_s < (S > 16 ? 8 : 2) || p.part_bytes(M, N) > part_bytes))) continue;
       double us = tile_time(ti, tiles * S, nk_s, group);
       if (S > 1) {
         us += (reduce ? 2.0 : 0.0) + 1.45e-6 * static_cast<double>(S * M * N);

@@ -515,7 +515,10 @@ def test_linear_ws_entries_cover_once(idx):
     (32, 8448, 4096, 128, 7), (16, 4096, 8192, 128, 1), (8, 4096, 14336, 128, 1), (16, 4096, 12288, 32, 1), (32, 4096, 4096, 128, 1),
     (40, 96, 192, 96, 1),  # a group that is no power of two: the workspace-free kernel
     (64, 256, 2048, 64, 16), (70, 1408, 1536, 32, 12), (50, 520, 2048, 256, 8), (256, 5120, 3072, 128, 3), (100, 515, 3072, 32, 16),
-    # more than 16 ranges only of nine stages or more; a split of little K for few columns
+    # groups of 64 and past 128 have rates of their own
+    (131, 3131, 2048, 256, 1), (87, 13092, 5568, 64, 4),
+    # more than 16 ranges only of eight stages or more; a split of little K for few columns
+    (48, 606, 13824, 512, 27),
     (20, 1536, 28672, 32, 32), (20, 2048, 18432, 128, 29), (40, 1024, 4096, 128, 16), (40, 64, 1024, 128, 8)])
 def test_linear_ws_split_bytes_is_what_the_call_writes(M, N, K, group, splits):
     """q4_linear_ws_split_bytes: the planes alone wherever the call adds no partials, else the planes (from a
