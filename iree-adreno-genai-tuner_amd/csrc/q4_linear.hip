@@ -1114,11 +1114,14 @@ bool swiglu_epilogue(int64_t M, int64_t N) {
 }
 
 // Calls of q4_linear_ws that one launch without planes or partials serves better: a few rows (q4_rows_wins;
-// short of the partials that the tiles need, all that the kernel takes), and K of at most two stages while its 64x64 tiles run at once, where the launch that splits x costs more than it
-// gives: 250x3560x128 7.8 -> 6.2 us, 33x256x128 6.4 -> 5.5 (two rounds of tiles, 700x3560x128: 12.7 | 14.9);
-// K 384 is past the line, 250x3560x384 10.3 | 11.4.
+// short of the partials that the tiles need, all that the kernel takes), and little K while its 64x64 tiles run
+// at once (two rounds, 700x3560x128: 12.7 us on the tiles | 14.9), where the launch that splits x costs more than
+// it gives: two stages, 250x3560x128 7.8 -> 6.2 us, 33x256x128 6.4 -> 5.5, and up to four where more than half of
+// the CUs have a tile: 512x2048x192 group 64 9.2 -> 7.9, 1024x1024x256 group 128 10.4 -> 9.2 (128 tiles,
+// 512x1024x256: 8.4 | 8.7; five stages, 512x2048x320 group 64: par).
 bool one_launch(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes) {
-  if (K <= 128 && ((M + 63) / 64) * ((N + 63) / 64) <= 512) return true;
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  if (tiles <= 512 && (K <= 128 || (K <= 256 && tiles > 128))) return true;
   return q4_rows_wins(M, N, K, group) ||
          (q4_rows_takes(M, K) && part_bytes < tile_plan(M, N, K, group, SIZE_MAX, true).part_bytes(M, N));
 }

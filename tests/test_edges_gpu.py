@@ -88,7 +88,8 @@ def test_linear_few_rows_on_tiles(dev, M, N, K, group):
 @pytest.mark.parametrize("M,N,K,group", [(33, 40, 128, 32), (100, 515, 3072, 32), (257, 256, 256, 128), (300, 1030, 2048, 64),
                                          (385, 260, 4096, 256), (513, 3072, 1024, 128), (640, 5120, 192, 64),
                                          (1024, 4100, 512, 128), (19, 819, 6144, 128), (35, 1225, 3904, 64), (250, 3560, 128, 128),
-                                         (700, 3560, 128, 32), (250, 3560, 384, 128), (33, 257, 64, 64), (257, 401, 4160, 32)])
+                                         (700, 3560, 128, 32), (250, 3560, 384, 128), (33, 257, 64, 64), (257, 401, 4160, 32), (1013, 1270, 192, 32),
+                                         (512, 2047, 256, 128), (512, 1025, 256, 64)])
 def test_linear_many_rows(dev, M, N, K, group):
     """q4_linear through its workspace: both pipelined tiles with ragged rows and columns, K splits (also of
     M N that is no multiple of four), the shortest K on both sides of the line to the one-launch kernel, an
