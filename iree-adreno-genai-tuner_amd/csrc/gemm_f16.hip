@@ -453,17 +453,18 @@ struct TileCfg {
   bool sp = false;  // software-pipelined substeps (gemm_f16_nt_kernel<..., true>)
 };
 // Explicit CDNA4 tile list. An entry keeps its index (gemm_f16_nt_cfg and the Q4_DBG_GEMM_TILE override select
-// by it): a new one takes the place of a removed one (3 and 4, once 64x96 and 128x64) or the end.
+// by it): a new one takes the place of a removed one (4, once 128x64) or the end.
 constexpr TileCfg kTiles[] = {
     {256, 256, 2, 4, 2, 64},        // 0: 8 waves of 128x64, 2 stages of K 64 (128 KB LDS)
     {128, 128, 2, 2, 2, 64},        // 1: 4 waves of 64x64, 2 stages (64 KB, two workgroups per CU)
-    {128, 128, 2, 2, 4, 64, true},  // 2: 4 waves of 64x64, 4 stages (128 KB), pipelined (entry 3 with one wave per
+    {128, 128, 2, 2, 4, 64, true},  // 2: 4 waves of 64x64, 4 stages (128 KB), pipelined (entry 8 with one wave per
                                     //    SIMD: for sweeps, the rule never takes it)
-    {128, 128, 4, 2, 4, 64, true},  // 3: 8 waves of 32x64, 4 stages (128 KB), pipelined
+    {64, 96, 2, 3, 4, 64, true},    // 3: 6 waves of 32x32, 4 stages (81 KB), pipelined
     {256, 128, 4, 2, 3, 64, true},  // 4: 8 waves of 64x64, 3 stages (144 KB), pipelined
     {64, 64, 2, 2, 4, 64},          // 5: 4 waves of 32x32, 4 stages (64 KB, two workgroups per CU)
     {128, 160, 2, 5, 4, 64, true},  // 6: 10 waves of 64x32, 4 stages (145 KB), pipelined
     {64, 128, 2, 4, 4, 64, true},   // 7: 8 waves of 32x32, 4 stages (96 KB), pipelined
+    {128, 128, 4, 2, 4, 64, true},  // 8: 8 waves of 32x64, 4 stages (128 KB), pipelined
 };
 constexpr int kSmallEntry = 5, kWideEntry = 2;  // the 64x64 tile; the 128x128 one that K splits are sized by below
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
@@ -482,9 +483,9 @@ constexpr size_t gemm_lds() {
   return GemmCfg<t.bm, t.bn, t.wgm, t.wgn, t.nst, t.bk>::kLds;
 }
 constexpr GemmFn kGemmFns[] = {gemm_fn<0>(), gemm_fn<1>(), gemm_fn<2>(), gemm_fn<3>(),
-                               gemm_fn<4>(), gemm_fn<5>(), gemm_fn<6>(), gemm_fn<7>()};
+                               gemm_fn<4>(), gemm_fn<5>(), gemm_fn<6>(), gemm_fn<7>(), gemm_fn<8>()};
 constexpr size_t kGemmLds[] = {gemm_lds<0>(), gemm_lds<1>(), gemm_lds<2>(), gemm_lds<3>(),
-                               gemm_lds<4>(), gemm_lds<5>(), gemm_lds<6>(), gemm_lds<7>()};
+                               gemm_lds<4>(), gemm_lds<5>(), gemm_lds<6>(), gemm_lds<7>(), gemm_lds<8>()};
 static_assert(sizeof(kGemmFns) / sizeof(kGemmFns[0]) == kNumTiles, "one kernel per tile entry");
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -538,37 +539,56 @@ struct GemmPlan {
 };
 
 // Estimated time (us) of `wgs` workgroups of `steps` K steps on entry ti: rounds of at most `cap` workgroups
-// (those that run at once), each costing its start and, per step, a time that grows with how many of them
-// load. Fitted (least squares of the relative error, median 4%) to 150 shapes of M 17-4096, N 64-5120, K
-// 64-8192 with splits of 1-16, graph replays over rotated operands on one MI355X. Entry 2 is left out.
-double tile_time(int ti, int64_t wgs, int64_t steps) {
+// (those that run at once), each costing its start and, per step, a time that grows with how many of them load
+// (from the 257th on a CU has two: `two`) and with `extra`, the further 128-byte lines that a row's 128 bytes of a
+// step touch: none where rows start on whole lines (K % 64 == 0), 7/8 where they start anywhere. Fitted (least
+// squares of the relative error, median 5-9% by entry) to 480 shapes of M 17-4096, N 256-32768, K 64-16384 from
+// 4 GFLOP on with splits of 1-16, graph replays over rotated operands on one MI355X. Without `extra` 64x128
+// was taken for long ragged K that other entries read better: 115x7028x6920 80 us, now 55; 387x2498x12488 111,
+// now 96. Entry 2 is left out.
+double tile_time(int ti, int64_t wgs, int64_t steps, int64_t K) {
   struct Rate {
-    double fixed, round, step, load;
+    double fixed, round, step, load, step_extra, load_extra, two;
     int cap;
   };
-  constexpr Rate kRates[kNumTiles] = {{8.9, 1.6, 1.346, 0.036, 256}, {5.7, 3.4, 0.575, 0.182, 512}, {0, 0, 0, 0, 0},
-                                      {4.5, 2.6, 0.443, 0.086, 256}, {6.2, 1.5, 0.740, 0.147, 256},
-                                      {3.2, 1.5, 0.322, 0.061, 512}, {5.1, 2.1, 0.568, 0.110, 256},
-                                      {3.5, 2.0, 0.354, 0.041, 256}};
+  constexpr Rate kRates[kNumTiles] = {
+      {7.9, 5.7, 1.344, 0.149, 0.207, 0.193, 0, 256},
+      {5.6, 6.1, 0.670, 0.153, 0.195, 0.067, 0.092, 512},
+      {},
+      {4.0, 2.3, 0.352, 0.045, 0.064, 0.038, 0, 256},
+      {6.3, 4.0, 0.708, 0.138, 0.111, 0.172, 0, 256},
+      {4.0, 1.9, 0.334, 0.000, 0.000, 0.075, 0.134, 512},
+      {5.4, 3.8, 0.544, 0.143, 0.159, 0.083, 0, 256},
+      {3.8, 2.3, 0.352, 0.070, 0.087, 0.036, 0, 256},
+      {4.8, 3.4, 0.426, 0.134, 0.147, 0.056, 0, 256}};
   const Rate& r = kRates[ti];
+  int64_t whole = 1;  // the largest power of two up to 64 that divides K
+  while (whole < 64 && K % (2 * whole) == 0) whole *= 2;
+  const double extra = 1.0 - static_cast<double>(whole) / 64.0;
+  auto step = [&](int64_t n) {
+    const double w = static_cast<double>(n) / 256.0;
+    return r.step + r.load * w + extra * (r.step_extra + r.load_extra * w) + (n > 256 ? r.two : 0.0);
+  };
   const int64_t full = wgs / r.cap, rest = wgs % r.cap;
   double us = r.fixed + static_cast<double>(full - (rest ? 0 : 1)) * r.round;
-  us += static_cast<double>(full * steps) * (r.step + r.load * r.cap / 256.0);
-  if (rest) us += static_cast<double>(steps) * (r.step + r.load * static_cast<double>(rest) / 256.0);
+  if (full) us += static_cast<double>(full * steps) * step(r.cap);
+  if (rest) us += static_cast<double>(steps) * step(rest);
   return us;
 }
 
 // The rule: latency-bound problems as above; else the cheapest entry by tile_time, with a K split of up to
 // 16 ranges of at least four steps where N % 4 == 0 and its partials fit `part_bytes` (their write, read and
-// launch: 3.3 us + 1.08 us per million; 5% in favour of no split, the estimate's error: 2048x3072x8192 in two
-// ranges was estimated at par and measured 121.8 us against 117.7). Against the fixed size rules before it
-// (us, same run): 256x3072x8192 28.9 -> 25.6, 512x3072x8192 83.9 -> 40.6, 512x5120x3072 39.1 -> 28.3,
-// 1024x3072x3072 38.9 -> 28.8, 3000x3000x3000 107 -> 92, 1536x1536x4096 47.3 -> 35.1, 256x16384x3072 38.1 ->
-// 34.0, 607x5172x64 8.0 -> 6.3; over the 150 shapes it is 1.6% off the best entry and split of each.
-// Measured and not in the list: whole-256-row tiles (256x64, 64x256, 256x32), 64x96 and 128x64, 4 waves of
-// 128x128 on 256x256 tiles (2 stages of K 64, or 4-5 stages of K 32) and of 64x128 / 128x64, 128x256, K
-// steps of 128, the plain schedule on the 4-stage tiles, the pipelined schedule on the 256x256 and the
-// two-workgroup 128x128 entries, and a ping-pong schedule of two 4-wave groups on 256x256.
+// launch: 3.3 us + 1.08 us per million; 5% in favour of no split, the estimate's error). Against the fixed size
+// rules before it (us, same run): 256x3072x8192 29.4 -> 27.6, 512x3072x8192 113 -> 43, 512x5120x3072 44 -> 31,
+// 1024x3072x3072 39.5 -> 29.7, 3000x3000x3000 110 -> 95, 1536x1536x4096 47 -> 35.5, 256x16384x3072 41.3 -> 40.0,
+// 607x5172x64 8.1 -> 6.5; over 960 shapes it is 1.3% off the best entry and split of each and 21% faster than
+// those rules (1% of the shapes more than 4% slower, the most 169x1840x9856 24.1 -> 27.3).
+// 64x96 is for problems without a split whose tiles of it make about one round: 175x6832x5600 56.6 us on 64x128,
+// 46.6 on it; 246x5382x5896 68.3 | 61.9.
+// Measured and not in the list: whole-256-row tiles (256x64, 64x256, 256x32), 128x64, 4 waves of 128x128 on
+// 256x256 tiles (2 stages of K 64, or 4-5 stages of K 32) and of 64x128 / 128x64, 128x256, K steps of 128, the
+// plain schedule on the 4-stage tiles, the pipelined schedule on the 256x256 and the two-workgroup 128x128
+// entries, and a ping-pong schedule of two 4-wave groups on 256x256.
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, size_t part_bytes) {
   const int ov = debug_override(Q4_DBG_GEMM_TILE);
   const bool forced = ov >= 0 && ov < kNumTiles;
@@ -588,7 +608,7 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, size_t part_bytes) {
       const int64_t nk_s = cdiv(nk, want), S = cdiv(nk, nk_s);
       const GemmPlan p{ti, {static_cast<int>(S), S > 1 ? static_cast<int>(nk_s) : 0}};
       if (S != want || (S > 1 && (N % 4 || M <= 1 || nk_s < 4 || p.bytes(M, N) > part_bytes))) continue;
-      double us = tile_time(ti, tiles * S, nk_s);
+      double us = tile_time(ti, tiles * S, nk_s, K);
       if (S > 1) us = 1.05 * (us + 3.3 + 1.08e-6 * static_cast<double>(S * M * N));
       if (us < best_us) best_us = us, best = p;
     }

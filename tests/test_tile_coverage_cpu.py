@@ -379,9 +379,9 @@ def test_tile_entries_keep_their_index():
     """A number noted from a sweep (gemm_f16_nt_cfg, the gemm_tile and linear_tile overrides) still names the
     tile that it named: entries stay where they are, also when others are removed or added."""
     gemm, lin = config_table("gemm"), config_table("linear_ws")
-    assert [gemm[i] for i in (0, 1, 2, 5, 6)] == [
-        (256, 256, 2, 4, 2, 64, 0), (128, 128, 2, 2, 2, 64, 0), (128, 128, 2, 2, 4, 64, 1), (64, 64, 2, 2, 4, 64, 0),
-        (128, 160, 2, 5, 4, 64, 1)]
+    assert [gemm[i] for i in (0, 1, 2, 3, 5, 6)] == [
+        (256, 256, 2, 4, 2, 64, 0), (128, 128, 2, 2, 2, 64, 0), (128, 128, 2, 2, 4, 64, 1), (64, 96, 2, 3, 4, 64, 1),
+        (64, 64, 2, 2, 4, 64, 0), (128, 160, 2, 5, 4, 64, 1)]
     assert [lin[i] for i in (1, 2)] == [(32, 64, 1, 2, 4, 2, 0), (64, 256, 2, 4, 4, 1, 1)]
 
 
