@@ -1067,7 +1067,8 @@ double tile_time(int ti, int64_t wgs, int64_t steps, int group) {
 // whole groups, at least two stages), whose partials fit `part_bytes`: their write and read cost 1.45 us per
 // million, the launch that adds them 2.0 us (none where the next kernel does it), and the estimate's error 5% in
 // favour of no split (none up to 12 us, where the fit is high for few columns: 40x64x1024 unsplit 11.8, split
-// 10.4). Past 16 ranges their sum takes a second round of loads: 40x1024x4096 16.5 us in 16 ranges, 21.5 in 32 of
+// 10.4; nor in a model step, whose T16 weights the pipelined tiles read in fewer lines than the fit's: 17 rows
+// through 2 layers of dim 4096, inter 14336 264 -> 254, as before the estimate). Past 16 ranges their sum takes a second round of loads: 40x1024x4096 16.5 us in 16 ranges, 21.5 in 32 of
 // two stages; long ranges gain by the CUs that 16 leave idle, 20x1536x28672 g32 50.2 -> 38.2, 20x2048x18432 29.7 ->
 // 27.6.
 // Against the 64x64 and 32x64 tiles that ran all of these before (us, with the x split): 512x5120x3072
@@ -1091,7 +1092,7 @@ LinPlan tile_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_bytes,
       double us = tile_time(ti, tiles * S, nk_s, group);
       if (S > 1) {
         us += (reduce ? 2.0 : 0.0) + 1.45e-6 * static_cast<double>(S * M * N);
-        if (us > 12.0) us *= 1.05;
+        if (us > 12.0 && reduce) us *= 1.05;
       }
       if (us < best_us) best_us = us, best = p;
     }

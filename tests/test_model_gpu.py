@@ -282,8 +282,8 @@ T16_DIMS = dict(hidden_size=1024, num_attention_heads=8, num_key_value_heads=4, 
 
 @pytest.mark.parametrize("cfg_kw,group,chunk,tile,plan", [
     # (tile entry, K ranges) of qkv, o, gate/up and down; entries 0 (128x256) and 2 (64x256) read T16
-    (T16_DIMS, 128, 256, None, ((1, 1), (1, 1), (2, 0), (2, 16))),  # gate/up: the SwiGLU epilogue
-    (T16_DIMS, 128, 128, None, ((1, 1), (2, 8), (2, 1), (2, 16))),
+    (T16_DIMS, 128, 256, None, ((1, 1), (2, 8), (2, 0), (2, 16))),  # gate/up: the SwiGLU epilogue
+    (T16_DIMS, 128, 128, None, ((2, 8), (2, 8), (2, 2), (2, 16))),
     (dict(T16_DIMS, intermediate_size=1024), 128, 100, None, ((2, 8),) * 4),  # every projection K-split
     (T16_DIMS, 128, 300, None, ((1, 1), (1, 1), (0, 1), (1, 1))),  # more than 256 rows: gate/up on 128x256
     (dict(hidden_size=256, num_attention_heads=64, num_key_value_heads=32, head_dim=128, intermediate_size=4096), 32, 300,
