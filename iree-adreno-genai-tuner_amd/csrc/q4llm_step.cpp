@@ -105,12 +105,16 @@ bool scales_on_words(const q4llm_model* m) {
 // the other path, whose projections are one launch each and read fp32 rows: what the tiled path fills with
 // padding and K splits costs more there. Measured (6 layers of dim 3072, inter 8192, group 128 | 4 layers of dim
 // 1024, inter 3072, group 32; tiled -> this, us): C = 2 527 -> 410 | 315 -> 183, C = 8 542 -> 462 | 325 -> 203,
-// C = 16 566 -> 533 | 337 -> 219. From 17 rows on while C dim <= 65536 (inter 4096: C = 17 535 -> 509, C = 24
-// 560 -> 558, C = 32 592 -> 605; dim 1024: C = 32 365 -> 262).
+// C = 16 566 -> 533 | 337 -> 219. That path's time grows with C K and the tiled one's hardly does, so up to C K =
+// 155648 for the largest K, half as much again for groups under 128, whose scales cost the tiles more (2 layers,
+// tiled | this, us; dim 4096, inter 14336: C = 10 254 | 245, 16 262 | 276, at group 32 16 295 | 285; dim 6144, inter
+// 16384: C = 8 372 | 373, 16 384 | 420), and up to the gate/up width from where on the tiles fill the chip without
+// K splits (dim 8192, inter 28672: C = 2 571 | 584, 8 574 | 645). From 17 rows on while C dim <= 65536 (6 layers,
+// inter 4096: C = 17 535 -> 509, C = 24 560 -> 558, C = 32 592 -> 605; dim 1024: C = 32 365 -> 262).
 bool prefill_planes(const q4llm_model* m, int C) {
-  const int D = m->dim, nq_w = m->n_heads * m->head_dim;
-  const bool few_rows = q4::q4_rows_takes(C, std::max(D, std::max(nq_w, m->inter))) &&
-                        (C <= 16 || static_cast<int64_t>(C) * D <= 65536);
+  const int D = m->dim, nq_w = m->n_heads * m->head_dim, kmax = std::max(D, std::max(nq_w, m->inter));
+  const bool few_rows = q4::q4_rows_takes(C, kmax) && (C <= 16 || static_cast<int64_t>(C) * D <= 65536) &&
+                        static_cast<int64_t>(C) * kmax <= (m->group < 128 ? 233472 : 155648) && m->inter <= 24576;
   return C > 1 && !few_rows && (m->group & (m->group - 1)) == 0 && linear_fits(D, m->group) &&
          linear_fits(nq_w, m->group) && linear_fits(m->inter, m->group) && scales_on_words(m);
 }

@@ -123,3 +123,21 @@ def test_debug_overrides_roundtrip_and_no_environment_reads():
         undef = subprocess.run([nm, "-D", "--undefined-only", str(LIB_PATH)], capture_output=True, text=True,
                                check=True).stdout
         assert "getenv" not in undef and "secure_getenv" not in undef
+
+
+@pytest.mark.parametrize("dim,heads,inter,group,c,tiles", [
+    (4096, 32, 14336, 128, 10, False), (4096, 32, 14336, 128, 11, True), (4096, 32, 14336, 32, 16, False),
+    (6144, 48, 16384, 256, 9, False), (6144, 48, 16384, 256, 16, True), (3072, 24, 8192, 128, 16, False),
+    (3072, 24, 8192, 128, 17, True), (2048, 16, 4096, 128, 32, False), (2560, 24, 4096, 128, 32, True),
+    (8192, 64, 28672, 128, 2, True)])
+def test_step_plan_few_rows_by_their_work(dim, heads, inter, group, c, tiles):
+    """Where a few rows stop being faster in one launch a projection: by rows times the largest K and the width of
+    gate/up, not by the number of rows alone."""
+    from q4llm.llama_q4 import _LayerC, _ModelC
+
+    layers = (_LayerC * 1)(_LayerC(*([FAKE] * 10)))
+    m = _ModelC(dim, 1, heads, 8, 128, inter, 1024, group, 128, 1e-5, FAKE, FAKE, FAKE, FAKE, FAKE,
+                C.cast(layers, C.c_void_p))
+    plan = (C.c_int * 8)()
+    assert LIB.raw("q4llm_step_plan")(C.byref(m), c, 128, plan) == 0
+    assert (list(plan) != [-1] * 8) == tiles
