@@ -243,7 +243,8 @@ int gemm_f16_nt_ws(const uint16_t* A, const uint16_t* B, uint16_t* C, int64_t M,
  * Attention over a KV bucket (reference: LlamaQ4.step, llama_q4.py:204-232)
  * ------------------------------------------------------------------------------------------- */
 
-/* Bytes of workspace attn_bucket needs for C query rows, n_q heads, head_dim hd, bucket L. */
+/* Bytes of workspace attn_bucket needs for C query rows, n_q heads, head_dim hd, bucket L; those of a
+ * prefill chunk (C > 1) also serve every smaller chunk of more than one row and every smaller bucket. */
 int attn_workspace_bytes(int C, int n_q, int n_kv, int hd, int L, size_t* bytes);
 
 /* GQA attention of C query rows at positions start[0] + c over k_cache/v_cache[:L]

@@ -31,6 +31,7 @@ struct AttnPlan {
   int S;         // keys per split
   int CB;        // query rows per workgroup
   int n_splits;  // ceil(L / S)
+  int ws_splits; // splits that a workspace is sized for (>= n_splits): no fewer for a larger C or L
   int n_cblk;    // ceil(C / CB)
   bool mfma;     // prefill chunk on the matrix cores (attn_prefill_mfma_kernel)
 };
@@ -41,6 +42,7 @@ AttnPlan plan_for(int C, int n_q, int n_kv, int L) {
   const int g = n_q / n_kv;
   AttnPlan p;
   p.mfma = false;
+  p.ws_splits = 0;
   if (C == 1) {
     p.CB = 1;
     p.S = L <= 1024 ? 32 : (L <= 2048 ? 64 : 128);
@@ -53,7 +55,11 @@ AttnPlan plan_for(int C, int n_q, int n_kv, int L) {
     p.CB = 32;
     const int64_t wgs = static_cast<int64_t>(n_kv) * (((C + 31) / 32 * g + 3) / 4);  // per split
     const int64_t want = std::max<int64_t>(1, 256 / wgs);
-    p.S = std::max(L <= 256 ? 64 : 128, static_cast<int>((L + 32 * want - 1) / (32 * want)) * 32);
+    // The workspace is sized by the least keys per split, whatever the chunk: fewer splits of a larger chunk
+    // would need less than a smaller one's, and a program keeps one workspace for its largest.
+    const int least = L <= 256 ? 64 : 128;
+    p.S = std::max(least, static_cast<int>((L + 32 * want - 1) / (32 * want)) * 32);
+    p.ws_splits = std::max((L + 127) / 128, std::min(4, (L + 63) / 64));
     const int ov = debug_override(Q4_DBG_ATTN_PS);  // sweep override: keys per split (a multiple of 32, <= 512)
     if (ov != Q4_DBG_UNSET && ov >= 32 && ov <= 512 && ov % 32 == 0) p.S = ov;
   } else {
@@ -61,6 +67,7 @@ AttnPlan plan_for(int C, int n_q, int n_kv, int L) {
     p.S = 64;
   }
   p.n_splits = (L + p.S - 1) / p.S;
+  p.ws_splits = std::max(p.ws_splits, p.n_splits);
   p.n_cblk = (C + p.CB - 1) / p.CB;
   return p;
 }
@@ -1019,18 +1026,21 @@ int attn_args(int C, int n_q, int n_kv, int hd, int L) {
   if (n_q % n_kv) return Q4_ERR_SHAPE;
   if (n_q / n_kv > kMaxQ) return Q4_ERR_UNSUPPORTED;
   if (hd != 64 && hd != 128) return Q4_ERR_UNSUPPORTED;
-  if (plan_for(C, n_q, n_kv, L).n_splits > 512) return Q4_ERR_UNSUPPORTED;  // combine holds <= 512 weights
+  if (plan_for(C, n_q, n_kv, L).ws_splits > 512) return Q4_ERR_UNSUPPORTED;  // combine holds <= 512 weights
   if (static_cast<int64_t>(L) * n_kv * hd * 2 >= (int64_t{1} << 31)) return Q4_ERR_SHAPE;
   return Q4_OK;
+}
+
+size_t partial_bytes(int C, int n_q, int hd, int splits) {
+  const size_t n = static_cast<size_t>(C) * n_q * splits;
+  return ml_floats(n) * sizeof(float) + n * hd * sizeof(float);
 }
 }  // namespace
 
 extern "C" int attn_workspace_bytes(int C, int n_q, int n_kv, int hd, int L, size_t* bytes) {
   if (!bytes) return Q4_ERR_NULL;
   if (int st = attn_args(C, n_q, n_kv, hd, L)) return st;
-  const AttnPlan p = plan_for(C, n_q, n_kv, L);
-  const size_t n = static_cast<size_t>(C) * n_q * p.n_splits;
-  *bytes = ml_floats(n) * sizeof(float) + n * hd * sizeof(float);
+  *bytes = partial_bytes(C, n_q, hd, plan_for(C, n_q, n_kv, L).ws_splits);
   return Q4_OK;
 }
 
@@ -1044,11 +1054,9 @@ int attn_bucket_impl(const float* q, int q_row_stride, const uint16_t* k_cache, 
   if (xh && (!xl || C == 1)) return Q4_ERR_SHAPE;
   if (int st = attn_args(C, n_q, n_kv, hd, L)) return st;
   if (q_row_stride < n_q * hd || q_row_stride % 4) return Q4_ERR_SHAPE;
-  size_t need = 0;
-  attn_workspace_bytes(C, n_q, n_kv, hd, L, &need);
-  if (workspace_bytes < need) return Q4_ERR_WORKSPACE;
-  if (!aligned(q, 16) || !aligned(k_cache, 16) || !aligned(v_cache, 16) || !aligned(workspace, 16)) return Q4_ERR_ALIGN;
   const AttnPlan p = plan_for(C, n_q, n_kv, L);
+  if (workspace_bytes < partial_bytes(C, n_q, hd, p.n_splits)) return Q4_ERR_WORKSPACE;
+  if (!aligned(q, 16) || !aligned(k_cache, 16) || !aligned(v_cache, 16) || !aligned(workspace, 16)) return Q4_ERR_ALIGN;
   float* ws_ml = static_cast<float*>(workspace);
   float* ws_o = ws_ml + ml_floats(static_cast<size_t>(C) * n_q * p.n_splits);
   const hipStream_t st = as_stream(stream);

@@ -141,3 +141,27 @@ def test_step_plan_few_rows_by_their_work(dim, heads, inter, group, c, tiles):
     plan = (C.c_int * 8)()
     assert LIB.raw("q4llm_step_plan")(C.byref(m), c, 128, plan) == 0
     assert (list(plan) != [-1] * 8) == tiles
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd", [(24, 8, 128), (4, 2, 64), (12, 12, 64), (64, 4, 64)])
+def test_attn_workspace_of_a_larger_call_serves_smaller_ones(n_q, n_kv, hd):
+    """A program sizes one workspace for its largest chunk and bucket: no smaller chunk or bucket asks for more."""
+    def need(c, l):
+        b = C.c_size_t(0)
+        assert LIB.raw("attn_workspace_bytes")(c, n_q, n_kv, hd, l, C.byref(b)) == 0
+        return b.value
+
+    for l in (100, 256, 300, 512, 2240, 2300, 4096):  # (C > 1: decode splits its keys finer)
+        sizes = [need(c, l) for c in range(2, 520)]
+        assert sizes == sorted(sizes)
+    for c in (2, 32, 100, 256):
+        sizes = [need(c, l) for l in range(1, 4100, 3)]
+        assert sizes == sorted(sizes)
+
+
+@pytest.mark.parametrize("c", [2, 32, 256, 2048])
+def test_attn_bucket_limit_is_the_same_for_every_chunk(c):
+    """Buckets past 65536 keys are refused for prefill chunks of any size."""
+    b = C.c_size_t(0)
+    call = lambda l: LIB.raw("attn_workspace_bytes")(c, 4, 2, 64, l, C.byref(b))
+    assert call(65536) == 0 and call(65537) == ERR["UNSUPPORTED"]
