@@ -538,29 +538,29 @@ struct GemmPlan {
   }
 };
 
-// Estimated time (us) of `wgs` workgroups of `steps` K steps on entry ti: rounds of at most `cap` workgroups
-// (those that run at once), each costing its start and, per step, a time that grows with how many of them load
-// (from the 257th on a CU has two: `two`) and with `extra`, the further 128-byte lines that a row's 128 bytes of a
-// step touch: none where rows start on whole lines (K % 64 == 0), 7/8 where they start anywhere. Fitted (least
-// squares of the relative error, median 5-9% by entry) to 480 shapes of M 17-4096, N 256-32768, K 64-16384 from
-// 4 GFLOP on with splits of 1-16, graph replays over rotated operands on one MI355X. Without `extra` 64x128
-// was taken for long ragged K that other entries read better: 115x7028x6920 80 us, now 55; 387x2498x12488 111,
-// now 96. Entry 2 is left out.
+// Estimated time (us) of `wgs` workgroups of `steps` K steps on entry ti, without the output: rounds of at most
+// `cap` workgroups (those that run at once), each costing its start and, per step, a time that grows with how many
+// of them load (from the 257th on a CU has two: `two`) and with `extra`, the further 128-byte lines that a row's 128
+// bytes of a step touch: none where rows start on whole lines (K % 64 == 0), 7/8 where they start anywhere. Fitted
+// (least squares of the relative error, by weight of how near an entry and split is to the best of its shape) to
+// 960 shapes of M 17-4096, N 256-32768, K 64-16384 from 4 GFLOP on with splits of 1-16, graph replays with operands
+// rotated past the caches and with resident ones on one MI355X. Without `extra` 64x128 was taken for long ragged K
+// that other entries read better: 115x7028x6920 80 us, now 55; 387x2498x12488 111, now 96. Entry 2 is left out.
 double tile_time(int ti, int64_t wgs, int64_t steps, int64_t K) {
   struct Rate {
     double fixed, round, step, load, step_extra, load_extra, two;
     int cap;
   };
   constexpr Rate kRates[kNumTiles] = {
-      {7.9, 5.7, 1.344, 0.149, 0.207, 0.193, 0, 256},
-      {5.6, 6.1, 0.670, 0.153, 0.195, 0.067, 0.092, 512},
+      {9.7, 7.3, 1.218, 0.437, 0.144, 0.158, 0, 256},
+      {6.4, 3.5, 0.522, 0.279, 0.225, 0.043, 0.013, 512},
       {},
-      {4.0, 2.3, 0.352, 0.045, 0.064, 0.038, 0, 256},
-      {6.3, 4.0, 0.708, 0.138, 0.111, 0.172, 0, 256},
-      {4.0, 1.9, 0.334, 0.000, 0.000, 0.075, 0.134, 512},
-      {5.4, 3.8, 0.544, 0.143, 0.159, 0.083, 0, 256},
-      {3.8, 2.3, 0.352, 0.070, 0.087, 0.036, 0, 256},
-      {4.8, 3.4, 0.426, 0.134, 0.147, 0.056, 0, 256}};
+      {3.7, 2.1, 0.356, 0.058, 0.025, 0.090, 0, 256},
+      {6.7, 4.3, 0.627, 0.346, 0.113, 0.057, 0, 256},
+      {3.9, 1.5, 0.331, 0.024, 0.000, 0.070, 0.102, 512},
+      {5.5, 2.9, 0.499, 0.254, 0.201, 0.007, 0, 256},
+      {3.7, 1.8, 0.342, 0.116, 0.001, 0.161, 0, 256},
+      {4.9, 2.4, 0.394, 0.208, 0.098, 0.097, 0, 256}};
   const Rate& r = kRates[ti];
   int64_t whole = 1;  // the largest power of two up to 64 that divides K
   while (whole < 64 && K % (2 * whole) == 0) whole *= 2;
@@ -576,13 +576,16 @@ double tile_time(int ti, int64_t wgs, int64_t steps, int64_t K) {
   return us;
 }
 
-// The rule: latency-bound problems as above; else the cheapest entry by tile_time, with a K split of up to
-// 16 ranges of at least four steps where N % 4 == 0 and its partials fit `part_bytes` (their write, read and
-// launch: 3.3 us + 1.08 us per million; 5% in favour of no split, the estimate's error). Against the fixed size
-// rules before it (us, same run): 256x3072x8192 29.4 -> 27.6, 512x3072x8192 113 -> 43, 512x5120x3072 44 -> 31,
-// 1024x3072x3072 39.5 -> 29.7, 3000x3000x3000 110 -> 95, 1536x1536x4096 47 -> 35.5, 256x16384x3072 41.3 -> 40.0,
-// 607x5172x64 8.1 -> 6.5; over 960 shapes it is 1.3% off the best entry and split of each and 21% faster than
-// those rules (1% of the shapes more than 4% slower, the most 169x1840x9856 24.1 -> 27.3).
+// The rule: latency-bound problems as above; else the cheapest entry by tile_time and the output's write (0.22 us
+// per million), with a K split of up to 16 ranges of at least four steps where N % 4 == 0 and its partials fit
+// `part_bytes` (their write, read and launch: 2.9 us + 0.75 us per million, and 2% in favour of no split). From 512
+// rows on it has to be 7% under the entry that the size alone gives (256x256 where its tiles fill the CUs, 128x160
+// where they make one round, else 128x128 with two workgroups per CU): such problems lie within the estimate's
+// error of each other, with operands resident or not (2048x3072x8192 on 256x128 114.6 | 121.7 us, on 128x128 112.4 |
+// 129.8). Against the size rules before it (us, same run): 256x3072x8192 29.3 -> 27.8, 256x5120x3072 22.7 -> 21.2,
+// 256x16384x3072 41.5 -> 39.9, 512x3072x8192 106 -> 43, 512x5120x3072 43.9 -> 31.2, 1024x3072x3072 39.5 -> 29.6,
+// 3000x3000x3000 109 -> 94, 1536x1536x4096 49.5 -> 35.4, 607x5172x64 8.1 -> 6.5; over another 960 shapes of the
+// same ranges, operands rotated or resident, 18% faster (0.8% of them more than 4% slower, the most 7%).
 // 64x96 is for problems without a split whose tiles of it make about one round: 175x6832x5600 56.6 us on 64x128,
 // 46.6 on it; 246x5382x5896 68.3 | 61.9.
 // Measured and not in the list: whole-256-row tiles (256x64, 64x256, 256x32), 128x64, 4 waves of 128x128 on
@@ -598,7 +601,10 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, size_t part_bytes) {
     return p.bytes(M, N) <= part_bytes ? p : GemmPlan{ti, {1, 0}};
   }
   GemmPlan best{kSmallEntry, {1, 0}};
-  double best_us = 1e30;
+  double best_us = 1e30, by_size_us = 0.0;
+  auto tiles_of = [&](int i) { return cdiv(M, kTiles[i].bm) * cdiv(N, kTiles[i].bn); };
+  const int by_size = M < 512 ? -1 : tiles_of(0) >= 256 ? 0 : tiles_of(6) >= 240 && tiles_of(6) <= 256 ? 6 : 1;
+  const double outputs = 1e-6 * static_cast<double>(M) * static_cast<double>(N);
   for (int ti = 0; ti < kNumTiles; ++ti) {
     if (ti == kWideEntry) continue;
     const TileCfg& t = kTiles[ti];
@@ -608,12 +614,13 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, size_t part_bytes) {
       const int64_t nk_s = cdiv(nk, want), S = cdiv(nk, nk_s);
       const GemmPlan p{ti, {static_cast<int>(S), S > 1 ? static_cast<int>(nk_s) : 0}};
       if (S != want || (S > 1 && (N % 4 || M <= 1 || nk_s < 4 || p.bytes(M, N) > part_bytes))) continue;
-      double us = tile_time(ti, tiles * S, nk_s, K);
-      if (S > 1) us = 1.05 * (us + 3.3 + 1.08e-6 * static_cast<double>(S * M * N));
+      double us = tile_time(ti, tiles * S, nk_s, K) + 0.22 * outputs;
+      if (S > 1) us = 1.02 * (us + 2.9 + 0.75 * static_cast<double>(S) * outputs);
+      if (S == 1 && ti == by_size) by_size_us = us;
       if (us < best_us) best_us = us, best = p;
     }
   }
-  return best;
+  return by_size >= 0 && best_us >= 0.93 * by_size_us ? GemmPlan{by_size, {1, 0}} : best;
 }
 
 // Whether gemm_f16_nt_ws takes this workspace: all that the split by size alone needs (problems under
