@@ -296,7 +296,7 @@ int argmax_f32(const float* logits, int64_t V, int32_t* out, void* workspace, si
  * ------------------------------------------------------------------------------------------- */
 
 /* Optional T16 copies (q4_t16_pack) of a weight for the decode GEMVs, also read by the prefill
- * GEMM's 64x256 tile: tiles and tile scales, both NULL when absent (decode and prefill then read
+ * GEMM's 64x256 and 128x256 tiles: tiles and tile scales, both NULL when absent (decode and prefill then read
  * the reference layout). wqkv takes Q4_PAIR_ROPE pairing, wgu Q4_PAIR_SWIGLU, wo, wdown and the
  * LM head Q4_PAIR_NONE. */
 typedef struct q4llm_t16 {

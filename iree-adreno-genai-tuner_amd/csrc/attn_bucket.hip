@@ -739,14 +739,18 @@ int launch_decode(const AttnPlan& p, int hd, int g, const float* q, const uint16
 // (ds_read_b64_tr_b16: 16 lanes read a 4 x 16 block and lane i receives column i), so neither P nor V is
 // transposed through registers or memory.
 //
-// What bounds it: the matrix cores run hi and lo (twice the useful flops) and the vector units share the
-// issue with them, so the softmax is kept short: the scale rides in the exponent's fma, exponents are
-// base 2 (m is in log2 units), only blocks that cross a row's position or L are masked, and the sums are
-// rescaled only when a maximum has grown by more than 2^8 (P then stays below 2^8, far inside fp16 hi + lo).
-// The partial (m, l, o) of each (row, head, split) goes to the workspace and the combine kernels merge
-// the splits.
-// Measured on one MI355X, 24/8 heads of 128, the combine included (us): C = 256 of 2048 keys 48.6 -> 30.0, of
-// 4096 91.8 -> 41, of 512 23.5 -> 19.7; 12/12 heads of 64, 256 of 2048 keys 16.7. Before: one 32-row block
+// What bounds it: a chain per block. The compiler puts a wait for every outstanding direct load in front of a
+// block's first transposing read, so the ring is drained once a block and the three stages in flight do not
+// outlast it (the counted wait before the barrier never binds); in a block, scores, softmax and P V follow each
+// other with two waves per SIMD to overlap. The matrix cores run hi and lo (twice the useful flops) and are busy
+// 26% of the cycles (C = 256 of 2048 keys), waves wait 30%. The softmax is kept short: the scale rides in the
+// exponent's fma, exponents are base 2 (m is in log2 units), only blocks that cross a row's position or L are
+// masked, and the sums are rescaled only when a maximum has grown by more than 2^8 (P then stays below 2^8, far
+// inside fp16 hi + lo). The partial (m, l, o) of each (row, head, split) goes to the workspace and the combine
+// kernels merge the splits.
+// Measured on one MI355X, 24/8 heads of 128, the last 256 of 2048 keys, the combine included: 48.8 -> 26.0 us a
+// call on one cache; in graph replays over three 51.2 -> 29.3, of 4096 keys 94.7 -> 41.1, rows 200-455 of 512 keys
+// 23.0 -> 19.0, 12/12 heads of 64, of 2048 keys 39.2 -> 17.6. Before: one 32-row block
 // and head group per workgroup, V transposed by 2-byte LDS stores, two barriers a block, a mask, an expf and a
 // rescaling on every block, and keys split 128 at a time whatever the chunk (51 MB of partials at 2048
 // keys). Of the 12.8 us of the kernel at 512 keys, writing the partials takes 4.4, the blocks 6.2, the

@@ -88,8 +88,8 @@ void linear_step_plan(int64_t M, int64_t N, int64_t K, int group, size_t part_by
 // With `deferred` not null, a K split leaves its partials in `part` unreduced and sets *deferred to the
 // number of splits (0 when the result went to y); the caller's next kernel then completes y.
 // The decode T16 copy of the same weight (q4_t16_pack: tiles, scales, and the pairing and head size it
-// was packed with), which the 64x256 tile reads instead of qw / sc when it takes the projection: its
-// 1 KB loads then touch 16 cache lines instead of 32.
+// was packed with), which the pipelined tiles (64x256 and 128x256) read instead of qw / sc when one of them takes
+// the projection: its 1 KB loads then touch 16 cache lines instead of 32.
 struct T16Src {
   const void* tiles;
   const uint16_t* scales;

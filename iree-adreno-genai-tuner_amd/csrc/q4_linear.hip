@@ -444,9 +444,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void q4_linear_ws_kernel(
     }
   }
   unsigned char* junk = lds + NST * G::kStage;
-  // Every step issues the same loads (steps past K load zeros into a free stage), so the number of
-  // vector-memory operations in flight is the same on every path: the exact waits below and the
-  // compiler's own waits for the scale registers then agree.
+  // Every step issues the same loads (steps past the range load its last stage again, into a free one), so the
+  // number of vector-memory operations in flight is the same on every path and the waits below are exact. The
+  // NST - 1 extra stages are real reads, mostly from L2: three beside the ten of a K range of 640.
   const int nk = K / 64;
   const int kt_begin = n_split > 1 ? ksp * nk_split : 0;
   const int kt_end = n_split > 1 ? min(nk, kt_begin + nk_split) : nk;
@@ -615,7 +615,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void q4_linear_ws_kernel(
     // first 16-k operands are then read while the last MFMAs of step l run. Step l issues the loads of
     // step l + NST - 1 into the buffer freed at the previous barrier (step l - 1's; buffer NST - 1 is
     // still unused at l = 0), spread over its first three 16-k steps, one between MFMAs. Every step
-    // issues the same kLPW loads (past kt_end: zeros), so the vmcnt counts below are constants.
+    // issues the same kLPW loads (past kt_end: the last stage's), so the vmcnt counts below are constants.
     static_assert(KS == 1, "the pipelined loop runs one wave group over all four 16-k steps");
     constexpr int KK = 4;
     const int nl = kt_end - kt_begin;
@@ -761,12 +761,12 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void q4_linear_ws_kernel(
     } else {
       for (int l = 0; l < nl; ++l) step_body(l, std::integral_constant<int, -1>{});
     }
-    wait_vmcnt<0>();  // the last steps' (zero) loads have landed before the waves exit
+    wait_vmcnt<0>();  // the loads issued past the range have landed before the waves exit
   }
 
   if constexpr (KS > 1) {
     // k-split: wave groups 1..KS-1 hand their sums to group 0 through LDS (the stage memory; the
-    // out-of-range loads of the last steps must land before it is reused). Layout [group][wave][tile]
+    // loads issued past the range must land before it is reused). Layout [group][wave][tile]
     // [e][lane]: every access is one 256-byte row.
     wait_vmcnt<0>();
     __syncthreads();

@@ -3,7 +3,7 @@
 //
 // The weights are read once, so the floor is their HBM time; what the 64-row tiles of q4_linear lose
 // here is rows padded to 64, too few workgroups and a serial chain of K steps. Instead:
-//   * a workgroup owns 16 NT columns and ALL of K: its waves take contiguous ranges of 128-k steps and
+//   * a workgroup owns 16 NT columns and ALL of K: its waves take 128-k steps in turn and
 //     meet in LDS at the end, so the chip is filled by columns x waves with no partials in memory and no
 //     second launch;
 //   * each wave loads what it multiplies straight into registers: per step and 16 columns one 16-byte load
@@ -14,6 +14,10 @@
 //   * group scales multiply the fp32 sums of each group (kG128: one group per 128-k step; otherwise
 //     every 32 k, so any group % 32 == 0 works).
 // Products, splits and accumulation are those of q4_linear: y = sum_g s_g sum_k (hi + lo)(n - 8) in fp32.
+// What bounds it is the latency of the loads (7x3072x3072: matrix cores busy 4% of the cycles, waves waiting 49%).
+// M <= 16: a wave's next step is loaded before the present one is multiplied, but in a branch, after which the
+// compiler waits for all loads, so in every other step the loads just issued too. M > 16: one step at a time, its
+// x loads sunk to their uses, several memory round trips a step; the time then grows with K (32x3072x8192 36 us).
 #include "q4_common.h"
 #include "q4_internal.h"
 
@@ -180,7 +184,7 @@ __global__ __launch_bounds__(MT == 1 && NT == 1 ? 1024 : 512) void q4_rows_kerne
     }
   };
 
-  if constexpr (MT == 1) {  // the next step's operands are in flight while this one is multiplied
+  if constexpr (MT == 1) {  // two steps' operands: the next one's loads are issued before this one is multiplied
     Step a, b;
     if (wave < steps) load(wave, a);
     for (int t = wave; t < steps; t += 2 * waves) {

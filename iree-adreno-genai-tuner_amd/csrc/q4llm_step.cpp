@@ -224,8 +224,8 @@ int step_impl(const q4llm_model* m, const int32_t* tokens, int C, const int32_t*
   } while (0)
 
   // Decode (C == 1), when the shapes take the vectorised GEMV (true for every BASELINE model), runs
-  // five kernels per layer: qkv GEMV with the input norm in its x staging and RoPE + the K/V cache
-  // writes in its epilogue; attention; o-projection + residual; gate/up GEMV with the post-attention
+  // six kernels per layer: qkv GEMV with the input norm in its x staging and RoPE + the K/V cache
+  // writes in its epilogue; attention (split and merge); o-projection + residual; gate/up GEMV with the post-attention
   // norm and SwiGLU in its epilogue; down-projection + residual; after the layers the LM head GEMV
   // takes the final norm in its x staging. Prefill uses the separate kernels.
   const bool fused = C == 1 && gemv_fusable(D, m->group);
@@ -239,7 +239,7 @@ int step_impl(const q4llm_model* m, const int32_t* tokens, int C, const int32_t*
   // decode GEMVs on the T16 copies where the model has them (Q4_DBG_NO_T16 set: the reference layout)
   const bool use_t16 = fused && !q4::debug_flag(Q4_DBG_NO_T16);
   auto has = [&](const q4llm_t16& t) { return use_t16 && t.tiles && t.scales; };
-  // prefill projections on the 64x256 tile read the same T16 copies (fewer cache lines per load)
+  // prefill projections on the 64x256 and 128x256 tiles read the same T16 copies (fewer cache lines per load)
   auto src = [&](const q4llm_t16& t, int pairing) {
     return q4::T16Src{t.tiles, static_cast<const uint16_t*>(t.scales), pairing, hd};
   };
